@@ -1050,3 +1050,37 @@ def test_wide_integer_weights_stay_exact(torch, ctx, wide):
     wt = ctx.weight_qconv(wc, zp=wzp)
     yc = ctx.qconv2d(_dev(torch, x), wt, x_zp=9, out_kind=L.QOUT_I32, pads=(1, 1, 1, 1)).cpu().numpy()
     np.testing.assert_array_equal(yc, O.conv_integer(x, wc, 9, wzp, pads=[1, 1, 1, 1]))
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 5, 8, 12, 16, 18])
+@pytest.mark.parametrize("dt", ["f32", "f16", "u8", "i32"])
+def test_ragged_output_rows_equal_aligned_ones(torch, ctx, dt, tile):
+    """Output rows that are no runs of aligned 16-byte chunks (an odd row
+    stride and a base one element off) hold the same bits as aligned rows, on
+    a partial last tile of every block tile, and nothing beside them changes."""
+    from oxionnx_amd import _lib as L
+    m, k, n = 261, 80, 323
+    rng = np.random.default_rng(tile)
+    if dt in ("f32", "f16"):
+        tdt = {"f32": torch.float32, "f16": torch.float16}[dt]
+        a = _dev(torch, rng.uniform(-1, 1, (m, k)).astype(np.float32)).to(tdt)
+        c = _dev(torch, rng.normal(0, 0.1, n).astype(np.float32)).to(tdt)
+        w = ctx.weight_gemm(rng.normal(0, 0.1, (k, n)).astype(np.float32), dtype=L.F32 if dt == "f32" else L.F16)
+        call = lambda out: ctx.gemm(a, w, c, act=L.ACT_RELU, out=out)   # noqa: E731
+    else:
+        tdt = {"u8": torch.uint8, "i32": torch.int32}[dt]
+        a = _dev(torch, rng.integers(0, 256, (m, k)).astype(np.uint8))
+        w = ctx.weight_qgemm(rng.integers(-127, 128, (k, n)).astype(np.int8), zp=0, scale=0.004)
+        kind = L.QOUT_U8 if dt == "u8" else L.QOUT_I32
+        call = lambda out: ctx.qgemm(a, w, a_zp=128, out_kind=kind, a_scale=0.02, y_scale=0.05, y_zp=128,   # noqa: E731
+                                     out=out)
+    wide = torch.zeros((m, 336), dtype=tdt, device="cuda")
+    odd = torch.full((m, 337), 7, dtype=tdt, device="cuda")
+    ctx.set_tile(tile)
+    try:
+        call(wide[:, :n])
+        call(odd[:, 1:1 + n])
+    finally:
+        ctx.set_tile(0)
+    assert torch.equal(odd[:, 1:1 + n], wide[:, :n])
+    assert bool((odd[:, 0] == 7).all()) and bool((odd[:, 1 + n:] == 7).all())
