@@ -106,11 +106,13 @@ struct OutMap {
   int ohw, P, Q;
   int vec;
   int splits;      // > 1: split-K over `splits` slices, partial sums in split_ws
-  void* split_ws;  // splits * Q * round_up(P, 4) accumulators (4 bytes each)
-  int batch;       // > 1: a batched launch of `batch` independent contractions (no split-K)
+  void* split_ws;  // batch * splits * Q * round_up(P, 4) accumulators (4 bytes each)
+  int batch;       // > 1: a batched launch of `batch` independent contractions
   int64_t zstride; // bytes between the batch slices' outputs
   int zsw;         // > 0: slice z's output starts at (z / zsw) * zrow + (z % zsw) * zstride
   int64_t zrow;
+  int rw;          // > 0: strided rows, element (i, j) at (i / ohw) * bstride + (i % ohw / rw) * rstride +
+  int64_t rstride; // (i % ohw % rw) * si + j * sj (a transposed convolution's phase over all images)
   int defer_reduce; // split-K: leave the partial sums in split_ws (the caller consumes them)
 };
 
@@ -135,12 +137,12 @@ inline int forced_splits() {
   }();
   return v;
 }
-inline int plan_splits(int P, int Q, int kc, int forced_tile, int auto_bs = 64) {
+inline int plan_splits(int P, int Q, int kc, int forced_tile, int auto_bs = 64, int batch = 1) {
   if (forced_tile != 0 && forced_tile != 10 && forced_tile != 11) return 1;
   if (forced_splits()) return forced_splits();
   const int64_t nk = (kc + 7) / 8;
   const int bs = forced_tile == 0 ? auto_bs : split_tile_size(P, Q, forced_tile);
-  const int64_t nb = (int64_t)((P + bs - 1) / bs) * ((Q + bs - 1) / bs);
+  const int64_t nb = (int64_t)((P + bs - 1) / bs) * ((Q + bs - 1) / bs) * batch;
   if (forced_tile != 0) return (int)std::max<int64_t>(2, std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1));
   if (nb >= 512 || nk < 16 || (nb >= 256 && nk < 32)) return 1;
   int64_t s = (512 + nb - 1) / nb;
@@ -156,15 +158,15 @@ inline int plan_splits(int P, int Q, int kc, int forced_tile, int auto_bs = 64) 
 struct SplitChoice {
   int splits, tile;
 };
-inline SplitChoice plan_split_tile(int P, int Q, int kc, int override_tile, bool mfma_f32) {
-  int s64 = plan_splits(P, Q, kc, override_tile);
+inline SplitChoice plan_split_tile(int P, int Q, int kc, int override_tile, bool mfma_f32, int batch = 1) {
+  int s64 = plan_splits(P, Q, kc, override_tile, 64, batch);
   // f32 on the 64x64 tile: slices of at least 12 k-stages (config 2b's
   // 128x768x3072, 24 stages: 2 slices 16.0 us against 3 slices 18.3)
   if (mfma_f32 && override_tile == 0 && !forced_splits() && s64 > 2)
     s64 = std::max(2, std::min(s64, (kc + 7) / 8 / 12));
   if (override_tile == 0 && mfma_f32 && s64 > 1) {   // only where the 64x64 plan splits too
-    const int s = plan_splits(P, Q, kc, 0, 128);
-    const int64_t nb = (int64_t)((P + 127) / 128) * ((Q + 127) / 128);
+    const int s = plan_splits(P, Q, kc, 0, 128, batch);
+    const int64_t nb = (int64_t)((P + 127) / 128) * ((Q + 127) / 128) * batch;
     if (s > 1 && nb * s >= 256) return {s, 11};
   }
   return {s64, override_tile};

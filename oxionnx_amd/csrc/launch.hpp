@@ -106,11 +106,12 @@ template <class OutT> struct FloatEpi {
   }
   __device__ __forceinline__ int out_bytes() const { return (int)sizeof(OutT); }
   __device__ __forceinline__ OutAddr addr() const { return out; }
-  __device__ __forceinline__ bool staged_ok(int bp) const {
+  // 16-byte chunks of output rows: no chunk straddles two images
+  __device__ __forceinline__ bool staged_ok() const {
     return out.stage && out.vec && ((uintptr_t)out.y % 16 == 0) && ((out.sj * (int64_t)sizeof(OutT)) % 16 == 0) &&
-           (out.bstride == 0 || out.ohw % bp == 0);
+           (out.bstride == 0 || (out.ohw * (int)sizeof(OutT) % 16 == 0 && out.bstride * (int64_t)sizeof(OutT) % 16 == 0));
   }
-  __device__ __forceinline__ bool staged_wide_ok(int bp) const { return sizeof(OutT) == 4 && staged_ok(bp); }
+  __device__ __forceinline__ bool staged_wide_ok() const { return sizeof(OutT) == 4 && staged_ok(); }
 
   struct PreI { float b[4]; };    // beta * bias per row (BIAS_I, BIAS_SCALAR), else -0
   struct PreJ { float b; };       // beta * bias per column (BIAS_J), else -0
@@ -230,13 +231,13 @@ struct QuantEpi {
   static constexpr bool kStageWide = true;   // int32 / f32 outputs stage as 4-byte elements
   __device__ __forceinline__ int out_bytes() const { return (out_kind == QOUT_U8 || out_kind == QOUT_I8) ? 1 : 4; }
   __device__ __forceinline__ OutAddr addr() const { return out; }
-  __device__ __forceinline__ bool staged_ok(int bp) const {
+  __device__ __forceinline__ bool staged_ok() const {
     return out.stage && (out_kind == QOUT_U8 || out_kind == QOUT_I8) && out.vec && ((uintptr_t)out.y % 16 == 0) &&
-           (out.sj % 16 == 0) && (out.bstride == 0 || out.ohw % bp == 0);
+           (out.sj % 16 == 0) && (out.bstride == 0 || (out.ohw % 16 == 0 && out.bstride % 16 == 0));
   }
-  __device__ __forceinline__ bool staged_wide_ok(int bp) const {
+  __device__ __forceinline__ bool staged_wide_ok() const {
     return out.stage && (out_kind == QOUT_I32 || out_kind == QOUT_F32) && out.vec && ((uintptr_t)out.y % 16 == 0) &&
-           (out.sj % 4 == 0) && (out.bstride == 0 || out.ohw % bp == 0);
+           (out.sj % 4 == 0) && (out.bstride == 0 || (out.ohw % 4 == 0 && out.bstride % 4 == 0));
   }
 
   // Per-channel terms of a weight channel, prepared once per block: cs the
@@ -436,8 +437,9 @@ inline hipError_t launch_reduce(const void* ws, int splits, int P, int Q, const 
   const int64_t groups = (int64_t)(Pp / 4) * Q;
   if (groups > 0x7fffffff) return hipErrorInvalidValue;   // the reduction indexes groups in 32 bits
   const unsigned grid = (unsigned)std::min<int64_t>((groups + 255) / 256, 65535 * 4);
-  hipLaunchKernelGGL((split_reduce_kernel<T, V, Epi>), dim3(grid), dim3(256), 0, st, reinterpret_cast<const T*>(ws),
-                     splits, P, Pp, Q, epi);
+  const int batch = epi.out.batch > 1 ? epi.out.batch : 1;
+  hipLaunchKernelGGL((split_reduce_kernel<T, V, Epi>), dim3(grid, 1, (unsigned)batch), dim3(256), 0, st,
+                     reinterpret_cast<const T*>(ws), splits, P, Pp, Q, epi);
   return hipGetLastError();
 }
 
@@ -450,11 +452,14 @@ inline hipError_t launch_split_on(const LX& lx, const LY& ly, const Epi& epi, in
   const int nP = (P + Tl::BP - 1) / Tl::BP, nQ = (Q + Tl::BQ - 1) / Tl::BQ;
   const int64_t nb = (int64_t)nP * nQ;
   if (nb <= 0) return hipSuccess;
-  if (nb > 0x7fffffff || splits > 65535 || !ws) return hipErrorInvalidValue;
+  const int batch = epi.out.batch > 1 ? epi.out.batch : 1;
+  if (nb > 0x7fffffff || splits > 65535 || batch > 65535 || !ws) return hipErrorInvalidValue;
+  if (epi.out.defer && batch > 1) return hipErrorInvalidValue;
   const int Pp = (P + 3) / 4 * 4;
   PartialEpi<T> pe{reinterpret_cast<T*>(ws), P, Pp, Q};
-  hipLaunchKernelGGL((mfma_gemm_kernel<O, Tl, LX, LY, PartialEpi<T>, XX, XY>), dim3((unsigned)nb, (unsigned)splits),
-                     dim3(Tl::kThreads), 0, st, lx, ly, pe, nP, nQ, kc, splits, tile_group_width());
+  hipLaunchKernelGGL((mfma_gemm_kernel<O, Tl, LX, LY, PartialEpi<T>, XX, XY>),
+                     dim3((unsigned)nb, (unsigned)splits, (unsigned)batch), dim3(Tl::kThreads), 0, st, lx, ly, pe, nP,
+                     nQ, kc, splits, tile_group_width());
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || epi.out.defer) return e;
   return launch_reduce<O>(ws, splits, P, Q, epi, st);
@@ -577,7 +582,6 @@ inline bool prefer_192x256(int P, int Q, int kc) {
 template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
 inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
                              int splits, void* split_ws, hipStream_t st) {
-  if (splits > 1 && epi.out.batch > 1) return hipErrorInvalidValue;   // one workspace: no split-K per slice
   if (splits > 1) {
     // OHIP_SPLIT_TILE=12/13/14 runs the slices on that deeper-pipelined tile (a measurement switch)
     static const int sv = [] { const char* e = std::getenv("OHIP_SPLIT_TILE"); return e ? std::atoi(e) : 0; }();
@@ -635,6 +639,8 @@ inline OutAddr make_out_addr(const OutMap& o) {
   a.P = o.P; a.Q = o.Q; a.vec = o.vec;
   a.batch = o.batch > 1 ? o.batch : 1; a.zstride = o.zstride;
   a.zsw = o.zsw; a.zrow = o.zrow;
+  a.rw = o.rw; a.rstride = o.rstride;
+  magic_div(a.rw > 0 ? a.rw : 1, &a.rw_mul, &a.rw_shift);
   a.defer = o.defer_reduce;
   return a;
 }

@@ -380,6 +380,8 @@ template <bool XOR> __device__ __forceinline__ u32x4 frag(u32x4 v) {
 // so the MFMA pipe is never left waiting on a barrier with no work queued.
 // Where the outputs go: element (i, j) sits at
 //   (i / ohw) * bstride + (i % ohw) * si + j * sj      (elements of `eb` bytes)
+// or, with rw > 0 (strided rows of an image: a transposed convolution's phase),
+//   (i / ohw) * bstride + (i % ohw / rw) * rstride + (i % ohw % rw) * si + j * sj,
 // with i / ohw computed as (i * ohw_mul) >> ohw_shift (exact for 0 <= i < 2^31,
 // magic_div below).  vec: si == 1 and every aligned run of four i is
 // contiguous and 4-element aligned in memory.
@@ -397,10 +399,23 @@ struct OutAddr {
   int zsw;           // > 0: slice z starts (z / zsw) * zrow + (z % zsw) * zstride bytes in
   int64_t zrow;
   int defer;         // host side: a split-K launch leaves its partial sums for the caller
+  int rw;            // > 0: an image's pixels are rows of rw, rstride elements apart
+  uint32_t rw_mul;
+  int rw_shift;
+  int64_t rstride;
   __device__ __forceinline__ int64_t row(int i) const {
     if (bstride == 0) return (int64_t)i * si;
     const int n = (int)(((uint64_t)(uint32_t)i * ohw_mul) >> ohw_shift);
-    return (int64_t)n * bstride + (int64_t)(i - n * ohw) * si;
+    const int r = i - n * ohw;
+    if (rw == 0) return (int64_t)n * bstride + (int64_t)r * si;
+    const int y = (int)(((uint64_t)(uint32_t)r * rw_mul) >> rw_shift);
+    return (int64_t)n * bstride + y * rstride + (int64_t)(r - y * rw) * si;
+  }
+  // bytes from slice 0's output to that of slice blockIdx.z
+  __device__ __forceinline__ int64_t slice_offset() const {
+    if (batch <= 1) return 0;
+    const int z = (int)blockIdx.z;
+    return zsw > 0 ? (int64_t)(z / zsw) * zrow + (int64_t)(z % zsw) * zstride : (int64_t)z * zstride;
   }
 };
 
@@ -467,11 +482,7 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   const int ibase = p0 + wp * Tl::TP * 32 + (lane >> 5) * 4;
   const int jbase = q0 + wq * Tl::TQ * 32 + (lane & 31);
   OutAddr out = epi.addr();
-  if (out.batch > 1) {
-    const int z = (int)blockIdx.z;
-    out.y += out.zsw > 0 ? (int64_t)(z / out.zsw) * out.zrow + (int64_t)(z % out.zsw) * out.zstride
-                         : (int64_t)z * out.zstride;
-  }
+  out.y += out.slice_offset();
 
   // the per-column epilogue terms, loaded once for all of this lane's rows
   typename Epi::PreJ pj[Tl::TQ];
@@ -486,8 +497,7 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   // Mode 1 stages the epilogue's narrow output (1 or 2 bytes); mode 2 stages
   // 4-byte outputs (int32, f32) when the tile's stage buffers hold them.
   // `ragged`: the output rows are not runs of aligned 16-byte chunks (an odd
-  // N or plane, a misaligned output, a strided transposed convolution), so
-  // the flush writes single elements, 64 consecutive i a wave.
+  // N or plane, a misaligned output, a strided transposed convolution).
   constexpr int EBN = Epi::kStageBytes > 0 ? Epi::kStageBytes : 1;
   // the row terms sit past the stage buffers, or (when both do not fit the
   // LDS) at the end of them, written once every load has landed
@@ -500,8 +510,8 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   int smode = 0;
   // the batch slice's own output must be 16-byte aligned too (the Epi checks slice 0's)
   const bool zaligned = ((uintptr_t)out.y % 16) == 0;
-  if constexpr (Epi::kStageBytes > 0) smode = zaligned && epi.staged_ok(Tl::BP) ? 1 : 0;
-  if constexpr (kWide) if (smode == 0 && zaligned && epi.staged_wide_ok(Tl::BP)) smode = 2;
+  if constexpr (Epi::kStageBytes > 0) smode = zaligned && epi.staged_ok() ? 1 : 0;
+  if constexpr (kWide) if (smode == 0 && zaligned && epi.staged_wide_ok()) smode = 2;
   const bool ragged = smode == 0;
   if constexpr (Epi::kStageBytes > 0) if (ragged && out.stage && epi.out_bytes() == EBN) smode = 1;
   if constexpr (kWide) if (ragged && out.stage && epi.out_bytes() == 4) smode = 2;
@@ -638,50 +648,59 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
     }
   };
   // The ragged flush.  Stored straight from the accumulators such outputs
-  // leave as single elements of 32 rows an instruction; from the staged rows
-  // a wave's store covers one run of 64 (i is a thread's constant, so its
-  // output offset is formed once).  96 x (197x64x197) f16 29.8 -> 19.4 us a
-  // call, 300x777x1001 bf16 11.4 -> 10.3, bit-identical; every ragged output
-  // that fits the stage buffers takes it (4-byte outputs of the largest
-  // tiles do not and leave from the accumulators).
-  auto flush_ragged = [&](auto ebc) __attribute__((always_inline)) {
-    constexpr int EB = decltype(ebc)::value;
+  // leave as single elements (or runs of four, out.vec) of 32 rows an
+  // instruction; from the staged rows a wave's store covers 64 units of one
+  // row (i is a thread's constant, so its output offset is formed once).
+  // 96 x (197x64x197) f16 29.8 -> 19.4 us a call, 300x777x1001 bf16 11.4 ->
+  // 10.3, bit-identical; every ragged output that fits the stage buffers
+  // takes it (4-byte outputs of the largest tiles do not and leave from the
+  // accumulators).
+  auto flush_ragged = [&](auto ebc, auto uc) __attribute__((always_inline)) {
+    constexpr int EB = decltype(ebc)::value, U = decltype(uc)::value, UPR = Tl::BP / U;
     constexpr int CPR = Tl::BP * EB / 16, SWZ = (CPR & -CPR) - 1;
     using E = std::conditional_t<EB == 4, uint32_t, std::conditional_t<EB == 2, uint16_t, uint8_t>>;
+    struct alignas(U * EB) Unit { E e[U]; };
     wait_lgkm0();
     barrier_only();
     auto put = [&](int li, int lj, int64_t row) __attribute__((always_inline)) {
       const int byte = li * EB;
-      const E v = *reinterpret_cast<const E*>(stg + lj * (Tl::BP * EB) + (((byte >> 4) ^ (lj & SWZ)) << 4) + (byte & 15));
-      *reinterpret_cast<E*>(out.y + (row + (int64_t)(q0 + lj) * out.sj) * EB) = v;
+      const Unit v =
+          *reinterpret_cast<const Unit*>(stg + lj * (Tl::BP * EB) + (((byte >> 4) ^ (lj & SWZ)) << 4) + (byte & 15));
+      char* dst = out.y + (row + (int64_t)(q0 + lj) * out.sj) * EB;
+      if (U == 1 || p0 + li + U <= out.P) {
+        *reinterpret_cast<Unit*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (p0 + li + u < out.P) reinterpret_cast<E*>(dst)[u] = v.e[u];
+      }
     };
-    if constexpr (Tl::kThreads % Tl::BP == 0) {
-      constexpr int JS = Tl::kThreads / Tl::BP;
-      const int li = t % Tl::BP;
+    if constexpr (Tl::kThreads % UPR == 0) {
+      constexpr int JS = Tl::kThreads / UPR;
+      const int li = t % UPR * U;
       if (p0 + li < out.P) {
         const int64_t row = out.row(p0 + li);
         const int jn = min(Tl::BQ, out.Q - q0);
 #pragma unroll 4
-        for (int lj = t / Tl::BP; lj < jn; lj += JS) put(li, lj, row);
+        for (int lj = t / UPR; lj < jn; lj += JS) put(li, lj, row);
       }
     } else {
-      for (int c = t; c < Tl::BQ * Tl::BP; c += Tl::kThreads) {
-        const int lj = c / Tl::BP, li = c - lj * Tl::BP;
+      for (int c = t; c < Tl::BQ * UPR; c += Tl::kThreads) {
+        const int lj = c / UPR, li = (c - lj * UPR) * U;
         if (q0 + lj < out.Q && p0 + li < out.P) put(li, lj, out.row(p0 + li));
       }
     }
   };
+  auto flush_any = [&](auto ebc) __attribute__((always_inline)) {
+    if (!ragged) flush(ebc);
+    else if (out.vec) flush_ragged(ebc, std::integral_constant<int, 4>{});
+    else flush_ragged(ebc, std::integral_constant<int, 1>{});
+  };
   if constexpr (Epi::kStageBytes > 0) {
-    if (smode == 1) {
-      if (ragged) flush_ragged(std::integral_constant<int, EBN>{});
-      else flush(std::integral_constant<int, EBN>{});
-    }
+    if (smode == 1) flush_any(std::integral_constant<int, EBN>{});
   }
   if constexpr (kWide) {
-    if (smode == 2) {
-      if (ragged) flush_ragged(std::integral_constant<int, 4>{});
-      else flush(std::integral_constant<int, 4>{});
-    }
+    if (smode == 2) flush_any(std::integral_constant<int, 4>{});
   }
 }
 
@@ -884,7 +903,8 @@ mfma_gemm_kernel(const LX lx, const LY ly, const Epi epi, int nP, int nQ, int kc
 
 // Split-K: slice s of the K loop stores its raw accumulators (f32, or i32
 // modulo 2^32) at ws[(s * Q + j) * Pp + i]; the reduction adds the slices in
-// slice order and hands each run of four sums to the real epilogue.
+// slice order and hands each run of four sums to the real epilogue.  A
+// batched launch (z) keeps its slices z after z.
 template <class T> struct PartialEpi {
   T* ws;
   int P, Pp, Q;
@@ -895,15 +915,15 @@ template <class T> struct PartialEpi {
   template <int EB, class A> __device__ __forceinline__ void finish_simple(const PreI&, A, uint32_t (&)[4]) const {}
   static constexpr int kStageBytes = 0;
   static constexpr bool kStageWide = false;
-  __device__ __forceinline__ bool staged_ok(int) const { return false; }
-  __device__ __forceinline__ bool staged_wide_ok(int) const { return false; }
+  __device__ __forceinline__ bool staged_ok() const { return false; }
+  __device__ __forceinline__ bool staged_wide_ok() const { return false; }
   struct PreJ {};
   __device__ __forceinline__ void load_i(PreI&, int) const {}
   __device__ __forceinline__ void load_j(PreJ&, int) const {}
   __device__ __forceinline__ int out_bytes() const { return 4; }
   __device__ __forceinline__ OutAddr addr() const {
     OutAddr o{};
-    o.y = reinterpret_cast<char*>(ws + (int64_t)blockIdx.y * Q * Pp);
+    o.y = reinterpret_cast<char*>(ws + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * Q * Pp);
     o.si = 1; o.sj = Pp; o.bstride = 0; o.ohw = 1; o.P = P; o.Q = Q; o.vec = 1;
     return o;
   }
@@ -923,7 +943,9 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const T* __restrict__
   const int groups = Pp / 4;
   const int64_t n = (int64_t)groups * Q;
   const int64_t slice = (int64_t)Q * Pp;   // elements per K slice
-  const OutAddr out = epi.addr();
+  OutAddr out = epi.addr();
+  out.y += out.slice_offset();
+  ws += (int64_t)blockIdx.z * splits * slice;
   for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n; g += (int64_t)gridDim.x * 256) {
     // n < 2^31 for every workspace the host sizes, so the index split is 32-bit
     const int gi = (int)g;

@@ -1841,24 +1841,37 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
       for (int64_t rx = 0; rx < sw; ++rx)
         max_rows = std::max<int64_t>(max_rows, ((oh - ry + sh - 1) / sh) * ((ow - rx + sw - 1) / sw));
     // Every phase in one launch, phase z = ry * sw + rx on the grid's z, when
-    // the phases share one filter allocation and one output grid and none
-    // runs split-K: the phase's pads, filter and output offset follow z.  A
-    // combined grid of 256+ blocks fills the chip without splitting; a
-    // forced split (tile 10 / 11, OHIP_SPLITS) keeps the per-phase launches.
-    const int64_t ohp0 = oh / sh, owp0 = ow / sw;
-    const int64_t blocks64 = ((ohp0 * owp0 + 63) / 64) * ((d->cout + 63) / 64) * sh * sw;
+    // the phases share one filter allocation and one output grid: the phase's
+    // pads, filter and output offset follow z, and so do the K slices of a
+    // grid too small to fill the chip (a forced split, tile 10 / 11 or
+    // OHIP_SPLITS, keeps the per-phase launches).  All images run in that
+    // launch too, one after another along the pixel rows (f32 3x142x9x9 ->
+    // 109 channels, formerly 12 split launches and their reductions: 170 ->
+    // 18 us; 40 shapes of 1-4 images: 2.2x in the mean); images of less than
+    // one 64-row tile keep a launch each (contraction_launches counts them
+    // so).
+    const int64_t ohp0 = oh / sh, owp0 = ow / sw, prow = ohp0 * owp0;
     const bool split_forced = ctx->tile_override == 10 || ctx->tile_override == 11 || forced_splits() != 0;
-    const bool one = w->ph_all && oh % sh == 0 && ow % sw == 0 && ohp0 > 0 && owp0 > 0 && ph_one_launch() &&
-                     !split_forced &&
-                     (blocks64 >= 256 ||
-                      plan_splits((int)(ohp0 * owp0), (int)d->cout, w->ph_all->kc, ctx->tile_override) == 1);
+    const bool one = w->ph_all && oh % sh == 0 && ow % sw == 0 && prow > 0 && ph_one_launch() && !split_forced &&
+                     d->n * prow <= INT_MAX / 2;
+    const int64_t joined = one && prow >= 64 ? d->n : 1;
     int max_splits = 1;
-    if (!one)
+    SplitChoice sc{1, ctx->tile_override};
+    if (one) {
+      const int64_t blocks64 = ((joined * prow + 63) / 64) * ((d->cout + 63) / 64) * sh * sw;
+      if (blocks64 < 256)
+        sc = plan_split_tile((int)(joined * prow), (int)d->cout, w->ph_all->kc, ctx->tile_override,
+                             d->dtype == OHIP_F32, (int)(sh * sw));
+      max_splits = sc.splits;
+    } else {
       for (auto* ph : w->phases)
         max_splits = std::max(max_splits, plan_splits((int)max_rows, (int)d->cout, ph->kc, ctx->tile_override));
+    }
     ScratchPlan plan;
     size_t ix = plan.add((size_t)(d->n * d->h * d->w * cp) * eb);
-    size_t iw = max_splits > 1 ? plan.add(split_ws_bytes((int)max_rows, (int)d->cout, max_splits)) : SIZE_MAX;
+    size_t iw = max_splits > 1 ? plan.add(one ? split_ws_bytes((int)(joined * prow), (int)d->cout, max_splits) * (size_t)(sh * sw)
+                                              : split_ws_bytes((int)max_rows, (int)d->cout, max_splits))
+                               : SIZE_MAX;
     rc = scratch_reserve(ctx, plan.total());
     if (rc) return rc;
     void* px = scratch_at(ctx, plan, ix);
@@ -1866,13 +1879,13 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
             "NCHW -> NHWC");
     if (one) {
       const ohip_weight* pa = w->ph_all;
-      for (int64_t n = 0; n < d->n; ++n) {
+      for (int64_t n = 0; n < d->n; n += joined) {
         Im2colOperand col{};
         col.base = static_cast<const char*>(px) + n * d->h * d->w * cp * eb;
         col.H = (int)d->h; col.W = (int)d->w; col.OH = (int)ohp0; col.OW = (int)owp0;
         col.KW = (int)pa->kw; col.cpc = (int)(cp / ce);
         col.sh = 1; col.sw = 1; col.dh = 1; col.dw = 1;
-        col.rows = (int)(ohp0 * owp0); col.kc = pa->kc;
+        col.rows = (int)(joined * prow); col.kc = pa->kc;
         col.xor_mask = 0; col.pad16 = pad16(ctx, 0);
         col.zpads = (int)(sh * sw);
         for (int64_t ry = 0; ry < sh; ++ry)
@@ -1888,13 +1901,14 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
         FloatOut o{};
         o.y = static_cast<char*>(y) + n * d->cout * oh * ow * eb;
         o.alpha = 1.0f; o.beta = 1.0f; o.bias = bias; o.bias_mode = BIAS_J; o.act = ACT_NONE;
-        o.si = sw; o.sj = oh * ow; o.bstride = sh * ow; o.ohw = (int)owp0;
-        o.P = (int)(ohp0 * owp0); o.Q = (int)d->cout; o.vec = 0;
-        o.splits = 1; o.split_ws = nullptr;
+        o.si = sw; o.sj = oh * ow; o.bstride = d->cout * oh * ow; o.ohw = (int)prow;
+        o.rw = (int)owp0; o.rstride = sh * ow;
+        o.P = col.rows; o.Q = (int)d->cout; o.vec = 0;
+        o.splits = sc.splits; o.split_ws = sc.splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
         o.batch = (int)(sh * sw); o.zsw = (int)sw; o.zrow = ow * eb; o.zstride = eb;   // phase (ry, rx) at ry * ow + rx
         DENSE_FITS_OR_DECLINE(wt, "ohip_conv_transpose2d");
         ctx->counters.contraction_launches++;
-        hipError_t e = run_conv_float(d->dtype, col, wt, true, o, ctx->tile_override, ctx->stream);
+        hipError_t e = run_conv_float(d->dtype, col, wt, true, o, sc.tile, ctx->stream);
         if (e != hipSuccess) return hip_fail(e, "ohip_conv_transpose2d phase launch");
       }
       return OHIP_OK;

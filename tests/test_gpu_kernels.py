@@ -1084,3 +1084,27 @@ def test_ragged_output_rows_equal_aligned_ones(torch, ctx, dt, tile):
         ctx.set_tile(0)
     assert torch.equal(odd[:, 1:1 + n], wide[:, :n])
     assert bool((odd[:, 0] == 7).all()) and bool((odd[:, 1 + n:] == 7).all())
+
+
+# one launch for every image (at least one 64-row tile a phase and image),
+# with and without K slices; (9, 7) is one row short of a tile
+@pytest.mark.parametrize("xs,cout,launches", [((3, 264, 9, 10), 37, 1), ((2, 264, 8, 8), 70, 1), ((3, 40, 11, 13), 5, 1),
+                                              ((2, 136, 9, 7), 33, 2)], ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f16"])
+def test_conv_transpose_joins_images(torch, ctx, xs, cout, launches, dt):
+    from oxionnx_amd import _lib as L
+    rng = np.random.default_rng(cout)
+    x = rng.uniform(-1, 1, xs).astype(np.float32)
+    w = rng.normal(0, 0.1, (xs[1], cout, 4, 4)).astype(np.float32)
+    b = rng.normal(0, 0.1, cout).astype(np.float32)
+    geo = dict(strides=[2, 2], pads=[1, 1, 1, 1])
+    tdt, ldt = (torch.float32, L.F32) if dt == "f32" else (torch.float16, L.F16)
+    wt = ctx.weight_conv_transpose(w, dtype=ldt, **geo)
+    xd, bd = _dev(torch, x).to(tdt), _dev(torch, b).to(tdt)
+    ctx.conv_transpose2d(xd, wt, bd, **geo)
+    ctx.reset_counters()
+    y = ctx.conv_transpose2d(xd, wt, bd, **geo)
+    assert ctx.counters()["contraction_launches"] == launches
+    want = torch.nn.functional.conv_transpose2d(
+        xd.cpu().double(), torch.from_numpy(w).to(tdt).double(), bd.cpu().double(), stride=2, padding=1).numpy()
+    assert _rel_err(y.float().cpu().numpy(), want) <= (F32_TOL if dt == "f32" else HALF_TOL)
