@@ -464,8 +464,8 @@ int ohip_reset_counters(ohip_ctx* ctx);
  *     rows take the whole-K halo kernel (no split-K) wherever its geometry
  *     allows (automatically from 256 blocks and 1.5 GFLOP up).
  * 18: 192x256 (8, two LDS stages, one block per CU).
- * The automatic choice splits K (on 64x64 tiles) when the 64x64 tiling gives
- * fewer than 256 blocks and K is at least 16 stages of 128 bytes. */
+ * The automatic choice takes the tile and the number of K slices with the
+ * least estimated time (plan_tiles). */
 int ohip_set_tile_override(ohip_ctx* ctx, int tile_id);
 
 #ifdef __cplusplus

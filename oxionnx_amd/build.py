@@ -34,7 +34,7 @@ def _compile(src, incremental=False):
     obj = os.path.join(OUT_DIR, os.path.splitext(src)[0] + ".o")
     if incremental and os.path.exists(obj):
         kern = ["mfma_core.hpp", "launch.hpp", "internal.hpp", "halo_conv.hpp", "norm_stats.hpp"]
-        local = {"ops.cpp": ["internal.hpp"], "dispatch.cpp": ["internal.hpp"],
+        local = {"ops.cpp": ["internal.hpp", "tile_plan.hpp"], "dispatch.cpp": ["internal.hpp"],
                  "aux_kernels.hip": kern, "nodes.hip": ["internal.hpp", "norm_stats.hpp"]}.get(src, kern + ["contract.inc"])
         deps = [os.path.join(CSRC, f) for f in [src] + local]
         if src.endswith(".cpp"):

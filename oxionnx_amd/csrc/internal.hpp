@@ -116,61 +116,6 @@ struct OutMap {
   int defer_reduce; // split-K: leave the partial sums in split_ws (the caller consumes them)
 };
 
-// Split-K plan.  The slices run on the 64x64 four-stage tile when its
-// tiling leaves the 256 CUs short of blocks (under one block per CU with at
-// least 16 stages of 128 bytes of K, or under two with at least 32); slices
-// keep at least 8 stages each and aim at two blocks per CU.  forced_tile
-// 10 / 11 force the split path on the 64x64 / 128x128 (eight-wave) tile; any
-// other forced tile disables it.  (The 128x128 slices measured slower on the
-// generator's resident NHWC convolutions, so the automatic plan keeps 64x64.)
-// Tile ids that name one unsplit block tile (launch.hpp); 10 and 11 force
-// split-K.
-inline bool plain_tile_id(int t) { return (t >= 1 && t <= 9) || (t >= 12 && t <= 14) || t == 16 || t == 18; }
-inline int split_tile_size(int, int, int forced_tile) { return forced_tile == 11 ? 128 : 64; }
-// OHIP_SPLITS=n (2..16) forces that many split-K slices wherever a split
-// plan is made (a measurement switch)
-inline int forced_splits() {
-  static const int v = [] {
-    const char* e = std::getenv("OHIP_SPLITS");
-    const int n = e ? std::atoi(e) : 0;
-    return n >= 2 && n <= 16 ? n : 0;
-  }();
-  return v;
-}
-inline int plan_splits(int P, int Q, int kc, int forced_tile, int auto_bs = 64, int batch = 1) {
-  if (forced_tile != 0 && forced_tile != 10 && forced_tile != 11) return 1;
-  if (forced_splits()) return forced_splits();
-  const int64_t nk = (kc + 7) / 8;
-  const int bs = forced_tile == 0 ? auto_bs : split_tile_size(P, Q, forced_tile);
-  const int64_t nb = (int64_t)((P + bs - 1) / bs) * ((Q + bs - 1) / bs) * batch;
-  if (forced_tile != 0) return (int)std::max<int64_t>(2, std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1));
-  if (nb >= 512 || nk < 16 || (nb >= 256 && nk < 32)) return 1;
-  int64_t s = (512 + nb - 1) / nb;
-  s = std::min<int64_t>(s, nk / 8);
-  s = std::min<int64_t>(s, 16);
-  return (int)std::max<int64_t>(s, 1);
-}
-// The split plan and the tile id to launch it with.  f32 contractions are
-// bound by the f32 MFMA rate, which the eight-wave 128x128 tile sustains
-// better than the 64x64 one (two accumulator chains per wave instead of
-// one), so their slices run on it (as forced tile 11) when that still gives
-// the chip a block per CU.
-struct SplitChoice {
-  int splits, tile;
-};
-inline SplitChoice plan_split_tile(int P, int Q, int kc, int override_tile, bool mfma_f32, int batch = 1) {
-  int s64 = plan_splits(P, Q, kc, override_tile, 64, batch);
-  // f32 on the 64x64 tile: slices of at least 12 k-stages (config 2b's
-  // 128x768x3072, 24 stages: 2 slices 16.0 us against 3 slices 18.3)
-  if (mfma_f32 && override_tile == 0 && !forced_splits() && s64 > 2)
-    s64 = std::max(2, std::min(s64, (kc + 7) / 8 / 12));
-  if (override_tile == 0 && mfma_f32 && s64 > 1) {   // only where the 64x64 plan splits too
-    const int s = plan_splits(P, Q, kc, 0, 128, batch);
-    const int64_t nb = (int64_t)((P + 127) / 128) * ((Q + 127) / 128) * batch;
-    if (s > 1 && nb * s >= 256) return {s, 11};
-  }
-  return {s64, override_tile};
-}
 inline size_t split_ws_bytes(int P, int Q, int splits) {
   return splits > 1 ? (size_t)splits * (size_t)Q * (size_t)((P + 3) / 4 * 4) * 4 : 0;
 }

@@ -536,47 +536,6 @@ inline hipError_t launch_wk(const HaloGeo& g, const Epi& epi, int P, int Q, void
   return pick(PartialEpi<float>{reinterpret_cast<float*>(ws), P, (P + 3) / 4 * 4, Q});
 }
 
-// Automatic choice (split-K is decided beforehand, plan_splits).  The
-// largest tile that still gives at least one block per CU (256 CUs); among
-// the smaller tiles, the two-stage 128x128 tile keeps two blocks resident
-// per CU and the four-stage 64x64 tile hides the load latency of the
-// narrowest problems.  A short K loop (few 128-byte stages) is dominated by
-// the prologue and the epilogue, which the resident 128x128 blocks overlap.
-inline int pick_tile(int P, int Q, int kc, int forced) {
-  if (plain_tile_id(forced)) return forced;
-  auto blocks = [&](int bp, int bq) { return (int64_t)((P + bp - 1) / bp) * ((Q + bq - 1) / bq); };
-  const int nk = (kc + 7) / 8;
-  if (nk <= 16) return blocks(128, 128) >= 256 ? 8 : 9;
-  // a long K and about one round of 128x128 tiles (config 3's second FFN
-  // GEMM, 4096x3072x768: 192 tiles): the four-stage eight-wave tile, one
-  // block per CU with deeper prefetch (int8 21.1 against 22.1 us for the
-  // two-stage tile; f16 1024x4096x4096 43.8 against 55.5, 768x4096x4096
-  // 38.5 against 52.0; f32 within 3 %)
-  if (blocks(128, 128) >= 192 && blocks(128, 128) < 320 && blocks(256, 256) < 256) return 12;
-  // the 256x256 tile with the X operand's loads two stages ahead
-  // (bit-identical; headline 312.0 -> 308.7 us, f16 8192^3 889.7 -> 868.6,
-  // bf16 863.6 -> 844.9; int8 8192^3 2423-2429 -> 2496-2508 TOPS and f32
-  // 4096x4096x11008 134.0 -> 136.1 TFLOP/s once its loop ran unrolled
-  // without K-tail selects)
-  if (blocks(256, 256) >= 256) return 16;
-  if (blocks(256, 128) >= 256) return P >= Q ? 3 : 4;
-  if (blocks(128, 128) >= 192) return 8;
-  return 9;
-}
-
-// Byte outputs (u8 / i8 requantised) of a short-K grid of more than two
-// rounds of 128x128 tiles (two blocks a CU) that the 192x256 tile covers in
-// one round of one block a CU: config 3's first FFN GEMM (4096x768 ->
-// 3072: 768 tiles of 128x128, 256 of 192x256) 22.6 -> 19.4 us.  Its
-// staged byte outputs fit the stage buffers; 4-byte outputs would leave
-// unstaged (MatMulInteger: 29.7 against 24.6 us) and keep the 128x128 tile.
-template <class Epi> inline bool byte_outputs(const Epi&) { return false; }
-inline bool byte_outputs(const QuantEpi& e) { return e.out_kind == QOUT_U8 || e.out_kind == QOUT_I8; }
-inline bool prefer_192x256(int P, int Q, int kc) {
-  auto blocks = [&](int bp, int bq) { return (int64_t)((P + bp - 1) / bp) * ((Q + bq - 1) / bq); };
-  return (kc + 7) / 8 <= 16 && blocks(128, 128) > 512 && blocks(192, 256) <= 256;
-}
-
 // XX / XY: the X / Y operand holds u8 activations that the MFMA reads as
 // int8 after XOR 0x80.
 template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
@@ -588,13 +547,11 @@ inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, 
     if (sv == 12) return launch_split_on<O, XX, XY, T128d4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
     if (sv == 13) return launch_split_on<O, XX, XY, T64d8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
     if (sv == 14) return launch_split_on<O, XX, XY, T128x4w4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-    if (split_tile_size(P, Q, tile) == 128)
+    if (tile == 11)
       return launch_split_on<O, XX, XY, T128w8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
     return launch_split_on<O, XX, XY, T64s4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
   }
-  int choice = pick_tile(P, Q, kc, tile);
-  if (tile == 0 && byte_outputs(epi) && prefer_192x256(P, Q, kc)) choice = 18;
-  switch (choice) {
+  switch (tile) {   // the caller's plan (plan_tiles)
     case 2: return launch_tile<O, XX, XY, T128>(lx, ly, epi, P, Q, kc, st);
     case 3: return launch_tile<O, XX, XY, T256x128>(lx, ly, epi, P, Q, kc, st);
     case 4: return launch_tile<O, XX, XY, T128x256>(lx, ly, epi, P, Q, kc, st);

@@ -20,6 +20,7 @@
 
 #include "../../include/ohip.h"
 #include "internal.hpp"
+#include "tile_plan.hpp"
 
 using namespace ohip;
 
@@ -106,13 +107,23 @@ struct DevPool {
   std::vector<std::pair<void*, size_t>> parked;
 };
 
+// The context's growable scratch.  A captured graph's kernels hold its address,
+// so the graph shares it: growth gives the context a new buffer and the old
+// one is freed with the last graph that was captured on it.
+struct ScratchBuf {
+  void* ptr = nullptr;
+  ~ScratchBuf() {
+    if (ptr) (void)hipFree(ptr);
+  }
+};
+
 struct ohip_ctx {
   int device = 0;
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
   ohip_tuning tuning{};
   int tile_override = 0;
-  void* scratch = nullptr;
+  std::shared_ptr<ScratchBuf> scratch;
   size_t scratch_bytes = 0;
   uint8_t* padtab = nullptr;  // 256 entries of 16 bytes: entry b is sixteen copies of byte b
   std::map<std::string, ohip_weight*> weights;
@@ -179,11 +190,12 @@ struct ScratchPlan {
 static int scratch_reserve(ohip_ctx* ctx, size_t bytes) {
   if (bytes <= ctx->scratch_bytes) return OHIP_OK;
   HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-  if (ctx->scratch) HIP_TRY(hipFree(ctx->scratch), "hipFree(scratch)");
-  ctx->scratch = nullptr;
+  ctx->scratch.reset();
   ctx->scratch_bytes = 0;
   size_t want = std::max<size_t>(bytes, size_t(1) << 20);
-  hipError_t e = dev_malloc(ctx, &ctx->scratch, want);
+  auto buf = std::make_shared<ScratchBuf>();
+  hipError_t e = dev_malloc(ctx, &buf->ptr, want);
+  if (e == hipSuccess) ctx->scratch = std::move(buf);
   if (e != hipSuccess) return fail(OHIP_E_NOMEM, std::string("scratch hipMalloc: ") + hipGetErrorString(e));
   ctx->scratch_bytes = want;
   return OHIP_OK;
@@ -192,7 +204,7 @@ static int scratch_reserve(ohip_ctx* ctx, size_t bytes) {
 static void* scratch_at(ohip_ctx* ctx, const ScratchPlan& p, size_t idx) {
   size_t off = 0;
   for (size_t i = 0; i < idx; ++i) off += p.sizes[i];
-  return static_cast<char*>(ctx->scratch) + off;
+  return static_cast<char*>(ctx->scratch->ptr) + off;
 }
 
 static void* plan_at(char* base, const ScratchPlan& p, size_t idx) {
@@ -236,7 +248,7 @@ static int call_scratch(ohip_ctx* ctx, size_t bytes, bool noalloc, char** base) 
   if (!noalloc) {
     int rc = scratch_reserve(ctx, bytes);
     if (rc) return rc;
-    *base = static_cast<char*>(ctx->scratch);
+    *base = ctx->scratch ? static_cast<char*>(ctx->scratch->ptr) : nullptr;
     return OHIP_OK;
   }
   if (bytes > kStaticScratchBytes)
@@ -321,7 +333,7 @@ extern "C" void ohip_ctx_destroy(ohip_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& kv : ctx->weights) weight_free(kv.second);
   for (auto* w : ctx->transients) weight_free(w);
-  if (ctx->scratch) (void)hipFree(ctx->scratch);
+  ctx->scratch.reset();
   if (ctx->padtab) (void)hipFree(ctx->padtab);
   for (auto& kv : ctx->tables) (void)hipFree(kv.second);
   for (auto& kv : ctx->consts) (void)hipFree(kv.second);
@@ -406,6 +418,7 @@ struct ohip_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<std::pair<void*, size_t>> held;
+  std::shared_ptr<ScratchBuf> scratch;
 };
 
 static void unpark_all(ohip_ctx* ctx, std::vector<std::pair<void*, size_t>>& v) {
@@ -444,6 +457,10 @@ extern "C" int ohip_graph_end(ohip_ctx* ctx, ohip_graph** out) {
   if (!out) return fail(OHIP_E_INVALID, "null out");
   auto* g = new ohip_graph();
   g->ctx = ctx;
+  {
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    g->scratch = ctx->scratch;
+  }
   hipError_t e = hipStreamEndCapture(ctx->stream, &g->graph);
   {
     std::lock_guard<std::mutex> lock(ctx->pool_mu);
@@ -1149,6 +1166,8 @@ static bool rows_direct(const void* a, int64_t k, int64_t ld, int eb, int trans)
 
 // ------------------------------------------------------------------ float GEMM
 static const int kMaxGemvM = 8;
+static PlanKind dense_kind(int dtype) { return dtype == OHIP_F32 ? PlanKind::DenseF32 : PlanKind::Dense; }
+static PlanKind conv_kind(int dtype) { return dtype == OHIP_F32 ? PlanKind::DenseF32 : PlanKind::Conv; }
 
 extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, const ohip_weight* b,
                          const void* c, void* y) {
@@ -1174,8 +1193,8 @@ extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, 
 
   ScratchPlan plan;
   size_t ia = direct ? SIZE_MAX : plan.add((size_t)(M * kp) * eb);
-  const SplitChoice sc = gemv ? SplitChoice{1, ctx->tile_override}
-                              : plan_split_tile((int)N, (int)M, b->kc, ctx->tile_override, d->dtype == OHIP_F32);
+  const TilePlan sc = gemv ? TilePlan{1, ctx->tile_override}
+                           : plan_tiles(dense_kind(d->dtype), (int)N, (int)M, b->kc, ctx->tile_override);
   const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, splits)) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
@@ -1399,7 +1418,7 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   // Groups whose output or input channel span is too narrow to fill an MFMA
   // tile (depthwise, and small groups) run the direct kernel on the NCHW
   // input; wider groups run on the MFMA engine (one launch with the group on
-  // the grid z, or a launch per group under split-K).  So do ungrouped
+  // the grid z).  So do ungrouped
   // convolutions of an NCHW input with under 32 taps x channels (an RGB stem,
   // whose 16-byte channel padding would multiply the staged bytes).  A long
   // reduction stays on the engine even for a few output channels: one
@@ -1506,9 +1525,16 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   const int hsplits = wk ? 0 : halo_plan(ctx, d, G, sw_, g, (int)(cp / ce), (int64_t)(sh_ * sw_ * cpt * eb));
   if (nhwc_pad && !hsplits && !wk)
     return fail(OHIP_DECLINED, "ohip_conv2d: a reflect / edge Pad on an NHWC input needs the halo-patch path");
-  const SplitChoice sc = wk ? SplitChoice{1, 0} : hsplits ? SplitChoice{hsplits, 0}
-                                 : plan_split_tile(sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override,
-                                                   d->dtype == OHIP_F32);
+  // groups share one launch (the group on the grid z)
+  TilePlan sc = wk        ? TilePlan{1, 0}
+                : hsplits ? TilePlan{hsplits, 0}
+                          : plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override,
+                                       (int)G);
+  // a static scratch too small for the slices' partial sums: no split
+  if (noalloc && !wk && !hsplits && sc.splits > 1 &&
+      split_ws_bytes(sP, sQ, sc.splits) * (size_t)G + (stage ? (size_t)(d->n * sh_ * sw_ * cpt) * eb : 0) + 512 >
+          kStaticScratchBytes)
+    sc = plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override, (int)G, false, false);
   const int splits = sc.splits;
   if (norm && splits == 1 && !wk) {   // counted again by the two-step path's plain call
     ctx->counters.dispatches--;
@@ -1525,7 +1551,7 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
                       (!norm->aff.residual || norm->aff.res_nhwc == (int)norm_nhwc) && aligned(y, 8 * eb) &&
                       aligned(norm->aff.residual, 8 * eb);
   const bool partials = splits > 1 || (wk && norm && !wk_mom);
-  size_t iw = partials ? plan.add(splits > 1 ? split_ws_bytes(sP, sQ, splits) : (size_t)sQ * ((sP + 3) / 4 * 4) * 4)
+  size_t iw = partials ? plan.add(splits > 1 ? split_ws_bytes(sP, sQ, splits) * (size_t)G : (size_t)sQ * ((sP + 3) / 4 * 4) * 4)
                        : SIZE_MAX;
   const size_t ity = wk_mom ? plan.add((size_t)(d->n * d->cout * ohw) * eb) : SIZE_MAX;
   const size_t imom = wk_mom ? plan.add((size_t)(d->n * d->cout * (ohw / 64)) * 2 * 4) : SIZE_MAX;
@@ -1599,11 +1625,10 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
     return OHIP_OK;
   }
 
-  // Groups without split-K run as one launch, group = blockIdx.z: the input
-  // channel chunks, the weight rows, the bias and the output channels of
-  // group z sit at fixed strides from group 0's.  Split plans share one
-  // workspace, so those run a launch per group.
-  const bool one_launch = G > 1 && G <= 65535 && splits == 1;
+  // Groups run as one launch, group = blockIdx.z: the input channel chunks,
+  // the weight rows, the bias, the output channels and the K slices of group
+  // z sit at fixed strides from group 0's.
+  const bool one_launch = G > 1 && G <= 65535;
   for (int64_t gi = 0; gi < (one_launch ? 1 : G); ++gi) {
     Im2colOperand col{};
     col.base = static_cast<const char*>(xin) + gi * cp * eb;
@@ -1782,6 +1807,9 @@ extern "C" int ohip_matmul(ohip_ctx* ctx, const ohip_matmul_desc* d, const void*
   ScratchPlan plan;
   size_t ib = plan.add((size_t)(d->b_batches * N * kp) * eb);
   size_t ia = a_direct ? SIZE_MAX : plan.add((size_t)(d->a_batches * M * kp) * eb);
+  const TilePlan sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce),
+                                 plain_tile_id(ctx->tile_override) ? ctx->tile_override : 0, (int)d->batch);
+  size_t iw = sc.splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
   if (rc) return rc;
   void* pb = scratch_at(ctx, plan, ib);
@@ -1800,12 +1828,12 @@ extern "C" int ohip_matmul(ohip_ctx* ctx, const ohip_matmul_desc* d, const void*
   o.y = y; o.si = 1; o.sj = N; o.bstride = 0; o.ohw = INT_MAX; o.P = (int)N; o.Q = (int)M;
   o.vec = N % 4 == 0 && aligned(y, 4 * eb);
   o.alpha = 1.0f; o.beta = 1.0f; o.bias = nullptr; o.bias_mode = BIAS_NONE; o.act = ACT_NONE;
-  o.splits = 1; o.split_ws = nullptr; o.batch = (int)d->batch; o.zstride = M * N * eb;
+  o.splits = sc.splits; o.split_ws = sc.splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
+  o.batch = (int)d->batch; o.zstride = M * N * eb;
   DENSE_FITS_OR_DECLINE(xo, "ohip_matmul");
   DENSE_FITS_OR_DECLINE(yo, "ohip_matmul");
   ctx->counters.contraction_launches++;
-  hipError_t e = run_dense_float(d->dtype, xo, yo, o, plain_tile_id(ctx->tile_override)
-                                                          ? ctx->tile_override : 0, ctx->stream);
+  hipError_t e = run_dense_float(d->dtype, xo, yo, o, sc.tile, ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "ohip_matmul launch");
   return OHIP_OK;
 }
@@ -1855,17 +1883,17 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
     const bool one = w->ph_all && oh % sh == 0 && ow % sw == 0 && prow > 0 && ph_one_launch() && !split_forced &&
                      d->n * prow <= INT_MAX / 2;
     const int64_t joined = one && prow >= 64 ? d->n : 1;
+    auto plan_rows = [&](int64_t rows, const ohip_weight* ph, int phases) {
+      return plan_tiles(conv_kind(d->dtype), (int)rows, (int)d->cout, ph->kc, ctx->tile_override, phases);
+    };
     int max_splits = 1;
-    SplitChoice sc{1, ctx->tile_override};
+    TilePlan sc{1, 0};
     if (one) {
-      const int64_t blocks64 = ((joined * prow + 63) / 64) * ((d->cout + 63) / 64) * sh * sw;
-      if (blocks64 < 256)
-        sc = plan_split_tile((int)(joined * prow), (int)d->cout, w->ph_all->kc, ctx->tile_override,
-                             d->dtype == OHIP_F32, (int)(sh * sw));
+      sc = plan_rows(joined * prow, w->ph_all, (int)(sh * sw));
       max_splits = sc.splits;
     } else {
-      for (auto* ph : w->phases)
-        max_splits = std::max(max_splits, plan_splits((int)max_rows, (int)d->cout, ph->kc, ctx->tile_override));
+      // (a phase's rows never exceed max_rows, but its plan may split more)
+      for (auto* ph : w->phases) max_splits = std::max(max_splits, plan_rows(max_rows, ph, 1).splits);
     }
     ScratchPlan plan;
     size_t ix = plan.add((size_t)(d->n * d->h * d->w * cp) * eb);
@@ -1935,12 +1963,13 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
           o.alpha = 1.0f; o.beta = 1.0f; o.bias = bias; o.bias_mode = BIAS_J; o.act = ACT_NONE;
           o.si = sw; o.sj = oh * ow; o.bstride = sh * ow; o.ohw = (int)owp;
           o.P = (int)(ohp * owp); o.Q = (int)d->cout; o.vec = 0;
-          const int splits = plan_splits(o.P, o.Q, ph->kc, ctx->tile_override);
-          o.splits = splits;
-          o.split_ws = splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
+          TilePlan pp = plan_rows(o.P, ph, 1);
+          if (pp.splits > max_splits) pp = plan_rows(max_rows, ph, 1);   // within the workspace
+          o.splits = pp.splits;
+          o.split_ws = pp.splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
           DENSE_FITS_OR_DECLINE(wt, "ohip_conv_transpose2d");
           ctx->counters.contraction_launches++;
-          hipError_t e = run_conv_float(d->dtype, col, wt, true, o, ctx->tile_override, ctx->stream);
+          hipError_t e = run_conv_float(d->dtype, col, wt, true, o, pp.tile, ctx->stream);
           if (e != hipSuccess) return hip_fail(e, "ohip_conv_transpose2d phase launch");
         }
     return OHIP_OK;
@@ -1986,7 +2015,9 @@ extern "C" int ohip_qgemm(ohip_ctx* ctx, const ohip_qgemm_desc* d, const void* a
   ScratchPlan plan;
   size_t ia = direct ? SIZE_MAX : plan.add((size_t)(M * kp));
   size_t ir = d->n_azp > 1 ? plan.add((size_t)M * 4) : SIZE_MAX;
-  const int splits = plan_splits((int)N, (int)M, b->kc, ctx->tile_override);
+  const int ob = (d->out_kind == OHIP_QOUT_I32 || d->out_kind == OHIP_QOUT_F32) ? 4 : 1;
+  const TilePlan sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4);
+  const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, splits)) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
   if (rc) return rc;
@@ -2008,7 +2039,6 @@ extern "C" int ohip_qgemm(ohip_ctx* ctx, const ohip_qgemm_desc* d, const void* a
   }
   QuantOut o{};
   o.y = y; o.si = 1; o.sj = ldy; o.bstride = 0; o.ohw = INT_MAX; o.P = (int)N; o.Q = (int)M;
-  const int ob = (d->out_kind == OHIP_QOUT_I32 || d->out_kind == OHIP_QOUT_F32) ? 4 : 1;
   o.vec = ldy % 4 == 0 && aligned(y, 4 * ob);
   o.w_on_i = 1; o.colsum = b->colsum; o.flip = b->flip; o.bias = nullptr;
   o.ca = shift - (d->a_zp ? d->a_zp[0] : 0); o.ca_rows = ca_rows;
@@ -2020,7 +2050,7 @@ extern "C" int ohip_qgemm(ohip_ctx* ctx, const ohip_qgemm_desc* d, const void* a
   o.splits = splits;
   o.split_ws = splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
   ctx->counters.contraction_launches++;
-  hipError_t e = run_dense_quant(x, yv, o, ctx->tile_override, ctx->stream);
+  hipError_t e = run_dense_quant(x, yv, o, sc.tile, ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "ohip_qgemm launch");
   return OHIP_OK;
 }
@@ -2115,7 +2145,8 @@ extern "C" int ohip_qconv2d(ohip_ctx* ctx, const ohip_qconv_desc* d, const void*
   const bool stage = d->in_layout == OHIP_NCHW;
   size_t ix = stage ? plan.add((size_t)(d->n * d->h * d->w * cpt)) : SIZE_MAX;
   const int sP = nchw_out ? (int)rows : (int)coutg, sQ = nchw_out ? (int)coutg : (int)rows;
-  const int splits = plan_splits(sP, sQ, w->kc, ctx->tile_override);
+  const TilePlan sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4);
+  const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes(sP, sQ, splits)) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
   if (rc) return rc;
@@ -2176,7 +2207,7 @@ extern "C" int ohip_qconv2d(ohip_ctx* ctx, const ohip_qconv_desc* d, const void*
     o.splits = splits;
     o.split_ws = splits > 1 ? scratch_at(ctx, plan, iw) : nullptr;
     ctx->counters.contraction_launches++;
-    hipError_t e = run_conv_quant(col, wt, col_on_x, o, ctx->tile_override, ctx->stream);
+    hipError_t e = run_conv_quant(col, wt, col_on_x, o, sc.tile, ctx->stream);
     if (e != hipSuccess) return hip_fail(e, "ohip_qconv2d launch");
   }
   return OHIP_OK;

@@ -1,0 +1,124 @@
+// The block tile and the K slices of a contraction on the MFMA engine, by
+// estimated time.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+
+namespace ohip {
+
+// Tile ids that name one unsplit block tile (launch.hpp); 10 and 11 force
+// split-K on the 64x64 / 128x128 (eight-wave) tile.
+inline bool plain_tile_id(int t) { return (t >= 1 && t <= 9) || (t >= 12 && t <= 14) || t == 16 || t == 18; }
+// OHIP_SPLITS=n (2..16) forces that many split-K slices wherever a split
+// plan is made (a measurement switch)
+inline int forced_splits() {
+  static const int v = [] {
+    const char* e = std::getenv("OHIP_SPLITS");
+    const int n = e ? std::atoi(e) : 0;
+    return n >= 2 && n <= 16 ? n : 0;
+  }();
+  return v;
+}
+
+// A block tile and the K slices it runs with (splits > 1: tile 10 or 11).
+struct TilePlan {
+  int splits, tile;
+};
+
+// What a block of a tile costs, in us: a stage of 128 bytes of K when its CU
+// is not short of bandwidth or MFMA rate (lat), a stage's share of the CU
+// when it is (bw: n resident blocks take max(lat, n * bw) a stage), and
+// everything outside the K loop (fix).  res: blocks a CU holds (LDS).
+struct TileCost {
+  int id, bp, bq, res;
+  float lat, bw, fix;
+};
+// The reduction of `s` slices of `mb` MB of partial sums in all.
+struct ReduceCost {
+  float fix, per_mb, per_slice;
+};
+enum class PlanKind { Dense, DenseF32, Conv };   // f16 / bf16 / int8 rows; f32 of any loader; im2col rows
+
+// The tile and the split of a contraction P x Q (x batch) over kc 16-byte
+// chunks, by the cost of every candidate.  The constants are a least-squares
+// fit to 178 shapes (M 12-4096, K 64-16384, N 64-11008; 1x1-5x5 convolutions
+// of 7-112 pixels; f16, f32, int8) timed on every tile and on 2-16 slices, graph
+// replay: the plan is within 1 % of the fastest candidate in the geometric
+// mean (worst 1.12x), where the rules it replaces, thresholds on the number
+// of blocks, were 8.8 % (dense), 11 % (f32) and 5 % (convolutions) from it,
+// up to 1.6x: f16 1024x1024x768 13.7 -> 9.0 us (split, now unsplit),
+// 1500x1024x2048 18.0 -> 12.7, 838x2688x2880 37 -> 24.
+// Grids of a round of 256x256 tiles and a long K take tile 16 outright: its
+// advantage there is the clock and the cache, which the stages' cost does
+// not show (4096x4096x11008 f16 291 us against 324 on tiles 3, 4 and 18).
+// The split is symmetric in P and Q (a convolution splits alike in NCHW and
+// NHWC output), so it is chosen without the one tile that is not square or
+// paired, 18 (whose 4-byte outputs do not fit its stage buffers: wide_out).
+inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_tile, int batch = 1,
+                           bool wide_out = false, bool may_split = true) {
+  static constexpr TileCost kDense[] = {{1, 64, 64, 4, .342f, .215f, .50f},   {9, 64, 64, 2, .287f, .178f, .78f},
+                                        {8, 128, 128, 2, .519f, .340f, 1.10f}, {12, 128, 128, 1, .373f, .373f, 1.93f},
+                                        {2, 128, 128, 1, .349f, .349f, 2.50f}, {3, 256, 128, 1, .475f, .475f, 2.80f},
+                                        {4, 128, 256, 1, .475f, .475f, 2.80f}, {16, 256, 256, 1, .902f, .887f, 4.36f},
+                                        {18, 192, 256, 1, .787f, .733f, 3.27f}};
+  static constexpr TileCost kF32[] = {{1, 64, 64, 4, .664f, .571f, .53f},     {9, 64, 64, 2, .654f, .565f, .98f},
+                                      {8, 128, 128, 2, 1.80f, 1.92f, 1.65f},  {12, 128, 128, 1, 2.04f, 2.04f, 1.68f},
+                                      {3, 256, 128, 1, 3.47f, 3.47f, 2.25f},  {4, 128, 256, 1, 3.47f, 3.47f, 2.25f},
+                                      {16, 256, 256, 1, 7.09f, 7.09f, 7.69f}};
+  static constexpr TileCost kConv[] = {{1, 64, 64, 4, .522f, .234f, .67f},    {9, 64, 64, 2, .386f, .254f, 1.17f},
+                                       {8, 128, 128, 2, .633f, .403f, 1.56f}, {12, 128, 128, 1, .510f, .510f, 2.15f},
+                                       {3, 256, 128, 1, .708f, .708f, 4.0f},  {4, 128, 256, 1, .708f, .708f, 4.0f}};
+  // (+ 1.5: a launch more also costs the host about 2 us, which small eager
+  // calls wait for: 5x960x1920 int8 pair 16.5 us, 18.8 with its second split)
+  const ReduceCost red = kind == PlanKind::Dense      ? ReduceCost{1.82f + 1.5f, .367f, .146f}
+                         : kind == PlanKind::DenseF32 ? ReduceCost{1.81f + 1.5f, .229f, .122f}
+                                                      : ReduceCost{1.21f + 1.5f, .321f, .121f};
+  const TileCost* tab = kind == PlanKind::Dense ? kDense : kind == PlanKind::DenseF32 ? kF32 : kConv;
+  const int ntab = kind == PlanKind::Dense      ? (int)(sizeof(kDense) / sizeof(TileCost))
+                   : kind == PlanKind::DenseF32 ? (int)(sizeof(kF32) / sizeof(TileCost))
+                                                : (int)(sizeof(kConv) / sizeof(TileCost));
+  const int64_t nk = std::max<int64_t>(1, ((int64_t)kc + 7) / 8);
+  if (plain_tile_id(override_tile)) return {1, override_tile};
+  if (override_tile != 0 && override_tile != 10 && override_tile != 11) {   // a forced path that does not apply here
+    override_tile = 0;
+    may_split = false;
+  }
+  if (forced_splits()) return {may_split ? forced_splits() : 1, override_tile ? override_tile : may_split ? 10 : 9};
+  if (override_tile != 0)
+    return {may_split ? (int)std::max<int64_t>(2, std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1)) : 1,
+            may_split ? override_tile : override_tile == 11 ? 8 : 9};
+  auto blocks = [&](int bp, int bq) { return (int64_t)((P + bp - 1) / bp) * ((Q + bq - 1) / bq) * batch; };
+  if (nk > 16 && blocks(256, 256) >= 256) return {1, 16};
+  auto time = [&](const TileCost& t, int64_t nb, int64_t stages) {
+    const int64_t ncu = (nb + 255) / 256, q = ncu / t.res, rem = ncu % t.res;
+    return t.fix * (float)(q + (rem ? 1 : 0)) +
+           (float)stages * ((float)q * std::max(t.lat, (float)t.res * t.bw) + (rem ? std::max(t.lat, (float)rem * t.bw) : 0.0f));
+  };
+  TilePlan best{1, 1};
+  float cost = INFINITY;
+  for (int i = 0; i < ntab; ++i) {
+    const TileCost& t = tab[i];
+    if (t.id == 18) continue;
+    if (wide_out && kind == PlanKind::Dense && t.bp * t.bq > 128 * 128) continue;   // unstaged 4-byte outputs
+    const float c = time(t, blocks(t.bp, t.bq), nk);
+    if (c < cost) { cost = c; best = {1, t.id}; }
+    if (!may_split || (t.id != 9 && t.id != 8)) continue;
+    for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
+      const int64_t per = (nk + s - 1) / s;
+      if (per < 2) break;
+      const float cs = time(t, blocks(t.bp, t.bq) * s, per) + red.fix + red.per_slice * (float)s +
+                       red.per_mb * (float)P * (float)Q * (float)batch * (float)s * 4e-6f;
+      if (cs < cost) { cost = cs; best = {s, t.id == 9 ? 10 : 11}; }
+    }
+  }
+  if (best.splits == 1 && kind == PlanKind::Dense && !wide_out) {
+    const TileCost& t = kDense[ntab - 1];
+    if (time(t, blocks(t.bp, t.bq), nk) < cost) best.tile = t.id;
+  }
+  return best;
+}
+
+}  // namespace ohip

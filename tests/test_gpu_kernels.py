@@ -1108,3 +1108,52 @@ def test_conv_transpose_joins_images(torch, ctx, xs, cout, launches, dt):
     want = torch.nn.functional.conv_transpose2d(
         xd.cpu().double(), torch.from_numpy(w).to(tdt).double(), bd.cpu().double(), stride=2, padding=1).numpy()
     assert _rel_err(y.float().cpu().numpy(), want) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+@pytest.mark.parametrize("a,b", [((2, 33, 2304), (2, 2304, 40)), ((3, 70, 1100), (3, 1100, 65)), ((5, 9, 4096), (1, 4096, 17))],
+                         ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f16"])
+def test_batched_matmul_with_k_slices(torch, ctx, a, b, dt):
+    """Few small slices over a long K: the K slices of every batch slice and
+    their reduction in one launch each, odd edges included."""
+    rng = np.random.default_rng(a[1])
+    tdt = torch.float32 if dt == "f32" else torch.float16
+    x = _dev(torch, rng.uniform(-1, 1, a).astype(np.float32)).to(tdt)
+    y = _dev(torch, rng.normal(0, b[1] ** -0.5, b).astype(np.float32)).to(tdt)
+    got = ctx.matmul(x, y).float().cpu().numpy()
+    want = np.matmul(x.cpu().double().numpy(), y.cpu().double().numpy())
+    assert _rel_err(got, want) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+def test_captured_scratch_outlives_growth(torch):
+    """A graph whose kernels use the context's scratch replays unchanged after
+    a larger call has given the context a new one."""
+    import ctypes
+
+    from oxionnx_amd import _lib as L
+    from oxionnx_amd.device import HipContext
+    ctx = HipContext(0)
+    rng = np.random.default_rng(3)
+    x = _dev(torch, rng.uniform(-1, 1, (1, 24, 20, 20)).astype(np.float32)).half()
+    w = ctx.weight_conv(rng.normal(0, 0.1, (40, 24, 3, 3)).astype(np.float32), dtype=L.F16)
+    y = torch.empty((1, 40, 20, 20), dtype=torch.float16, device="cuda")
+    ctx.conv2d(x, w, pads=(1, 1, 1, 1), out=y)
+    want = y.clone()
+    torch.cuda.synchronize()
+    g = ctypes.c_void_p()
+    L.check(L.lib().ohip_graph_begin(ctx.h))
+    ctx.conv2d(x, w, pads=(1, 1, 1, 1), out=y)
+    L.check(L.lib().ohip_graph_end(ctx.h, ctypes.byref(g)))
+    allocs = ctx.counters()["device_allocs"]
+    big = torch.zeros((4, 64, 128, 128), dtype=torch.float16, device="cuda")
+    wb = ctx.weight_conv(rng.normal(0, 0.1, (16, 64, 3, 3)).astype(np.float32), dtype=L.F16)
+    ctx.conv2d(big, wb, pads=(1, 1, 1, 1))
+    assert ctx.counters()["device_allocs"] > allocs
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        L.check(L.lib().ohip_graph_launch(g))
+        ctx.sync()
+        assert torch.equal(y, want)
+    L.lib().ohip_graph_destroy(g)
+    ctx.close()
