@@ -1266,6 +1266,125 @@ conv_dw3_kernel(const T* __restrict__ x, const T* __restrict__ w, const T* __res
   }
 }
 
+// Depthwise 3x3 from registers: a thread takes V outputs of R consecutive
+// output rows, loads the NR input rows it needs as one run of NV elements
+// each (whole dwords, shifted by a half where a 2-byte run starts in the
+// middle of one, all before the first sum), and slides down them.  No LDS, no barrier, and enough threads at every size.  The last
+// strip of a row ends with the row (overlapping its neighbour, which writes
+// the same values), so a run leaves the image by at most one element on
+// either side: that element is the neighbouring row's, replaced by zero, and
+// its tap's weight is zeroed too (a skipped tap adds nothing whatever the
+// weight holds); only the runs at the tensor's two ends load element by
+// element.  Taps in (ky, kx) order as conv_direct_kernel, by fused
+// multiply-adds (one rounding less a tap).  Bound: HBM on large planes (f32
+// 5.3 TB/s at 256 planes of 224x224, f16 3.0), the launch on small ones.
+struct DwStrip {
+  int strips, groups;   // V-wide strips a row, R-row groups a plane
+  uint32_t strip_mul, group_mul, cout_mul;
+  int strip_shift, group_shift, cout_shift;
+  int threads;
+};
+
+template <class T, int S, int V, int R>
+__global__ void __launch_bounds__(256)
+conv_dw3_strip_kernel(const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ y,
+                      DirectConvArgs a, DwStrip g) {
+  constexpr int NR = (R - 1) * S + 3, NV = (V - 1) * S + 3;
+  const int tid = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (tid >= g.threads) return;
+  auto udiv = [](int i, uint32_t mul, int shift) { return (int)(((uint64_t)(uint32_t)i * mul) >> shift); };
+  const int q = udiv(tid, g.strip_mul, g.strip_shift), strip = tid - q * g.strips;
+  const int plane = udiv(q, g.group_mul, g.group_shift), grp = q - plane * g.groups;
+  const int co = plane - udiv(plane, g.cout_mul, g.cout_shift) * a.cout;
+  const int ox0 = min(strip * V, a.OW - V), oy0 = grp * R;
+  const int ix0 = ox0 * S - a.pl, iy0 = oy0 * S - a.pt;
+  const int64_t total = (int64_t)a.N * a.cout * a.H * a.W;
+  constexpr int NW = sizeof(T) == 4 ? NV : (NV + 2) / 2;   // dwords that hold a run from the dword it starts in
+  struct Run { T e[2 * NW]; };
+  struct Words { uint32_t w[NW]; };
+  Run raw[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int iy = min(max(iy0 + r, 0), a.H - 1);
+    const int64_t at = ((int64_t)plane * a.H + iy) * a.W + ix0;
+    if (sizeof(T) == 4 ? at >= 0 && at + NV <= total : at >= 1 && at + 2 * NW <= total) {
+      const uintptr_t p = (uintptr_t)(x + at);
+      Words v;
+      __builtin_memcpy(&v, reinterpret_cast<const void*>(p & ~(uintptr_t)3), sizeof(Words));
+      if constexpr (sizeof(T) == 2) {
+        const uint32_t sh = (uint32_t)(p & 2) * 8;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) v.w[k] = __builtin_amdgcn_alignbit(k + 1 < NW ? v.w[k + 1] : 0u, v.w[k], sh);
+      }
+      __builtin_memcpy(&raw[r], &v, sizeof(Words));
+    } else {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) raw[r].e[j] = at + j >= 0 && at + j < total ? x[at + j] : T(0);
+    }
+  }
+  const bool left = ix0 < 0, right = ix0 + NV > a.W;
+  float wk[9], wl[3], wr[3];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) wk[k] = to_f32(w[(int64_t)co * a.ldw + k * a.cpg]);
+#pragma unroll
+  for (int ky = 0; ky < 3; ++ky) {
+    wl[ky] = left ? 0.0f : wk[ky * 3];
+    wr[ky] = right ? 0.0f : wk[ky * 3 + 2];
+  }
+  const float bv = bias ? to_f32(bias[co]) : 0.0f;
+  float v[NR][NV];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[r][j] = to_f32(raw[r].e[j]);
+    v[r][0] = left ? 0.0f : v[r][0];
+    v[r][NV - 1] = right ? 0.0f : v[r][NV - 1];
+  }
+  T* yp = y + ((int64_t)plane * a.OH + oy0) * a.OW + ox0;
+#pragma unroll
+  for (int o = 0; o < R; ++o) {
+    if (oy0 + o >= a.OH) break;
+    float acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+#pragma unroll
+    for (int ky = 0; ky < 3; ++ky) {
+      if ((unsigned)(iy0 + o * S + ky) < (unsigned)a.H) {
+#pragma unroll
+        for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            const float k = e == 0 && kx == 0 ? wl[ky] : (e == V - 1 && kx == 2 ? wr[ky] : wk[ky * 3 + kx]);
+            acc[e] = __builtin_fmaf(v[o * S + ky][e * S + kx], k, acc[e]);
+          }
+      }
+    }
+    struct Outs { T e[V]; } out;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      float r = acc[e];
+      if (bias) r = r + bv;
+      out.e[e] = from_f32<T>(activate_t<T>(r, a.act, a.lo, a.hi));
+    }
+    __builtin_memcpy(yp + (int64_t)o * a.OW, &out, sizeof(Outs));
+  }
+}
+
+// The strip width of a depthwise 3x3 for conv_dw3_strip_kernel, 0 where its
+// geometry does not hold: NCHW out, zero padding, strides 1 or 2, rows at
+// least a strip long whose runs leave the image by at most one element.
+// Eight-wide strips unless their overlap at the row's end costs more than the
+// wider runs save.
+inline int dw3_strip(const DirectConvArgs& a, int elem_bytes) {
+  if (!(a.cg == 1 && a.coutg == 1 && a.KH == 3 && a.KW == 3 && a.dh == 1 && a.dw == 1 && a.sh == a.sw &&
+        (a.sh == 1 || a.sh == 2) && a.pad_mode == 0 && !a.nhwc_out && a.pl >= 0 && a.pl <= 1))
+    return 0;
+  if ((a.OW - 1) * a.sh + 3 - a.pl - a.W > 1) return 0;
+  const int n8 = (a.OW + 7) / 8 * 8, n4 = (a.OW + 3) / 4 * 4;
+  if (elem_bytes == 2 && a.OW >= 8 && n8 * 7 <= n4 * 8) return 8;
+  return a.OW >= 4 ? 4 : 0;
+}
+
 // Output rows per band of the depthwise kernel (from 2^18 outputs): bands small enough for
 // about five blocks per CU (a block is a short serial chain of window load,
 // sums and stores; 128 blocks of 36 rows ran 9.6 us on 64 planes of 56x56),
@@ -1295,6 +1414,53 @@ hipError_t run_conv_direct(int dtype, const void* x, const void* w, const void* 
                            const DirectConvArgs& a, hipStream_t st) {
   const int64_t total = (int64_t)a.N * a.cout * a.OH * a.OW;
   if (total <= 0) return hipSuccess;
+  if (int strip = dw3_strip(a, dtype == DT_F32 ? 4 : 2)) {
+    // Wide strips from 2^17 threads up, two rows a thread (sharing the rows
+    // they read) from 2^19: below, more and shorter threads win, and more
+    // rows never do, since every wave then loads, sums and stores in step
+    // (f16, graph replay, against the band kernel or one thread an output:
+    // 1024 planes of 56x56 13.5 -> 7.2 us (8.2 four wide), 256 of 224x224
+    // 31 -> 16.9 (17.9 one row, 19.4 four), 32 of 112x112 6.4 -> 3.7 (4.2
+    // eight wide), 8192 of 7x7 19.9 -> 3.9; f32 1024 of 56x56 13.6 -> 7.8
+    // (8.2 one row)).
+    auto count = [&](int v, int r) {
+      return (int64_t)a.N * a.cout * ((a.OW + v - 1) / v) * ((a.OH + r - 1) / r);
+    };
+    if (strip == 8 && count(8, 1) < (1 << 17)) strip = 4;
+    const int R = count(strip, 1) < (1 << 19) ? 1 : 2;
+    const int64_t threads = count(strip, R);
+    if (threads <= 0x7fffff00) {
+      DwStrip g{};
+      g.strips = (a.OW + strip - 1) / strip; g.groups = (a.OH + R - 1) / R;
+      g.threads = (int)threads;
+      magic_div(g.strips, &g.strip_mul, &g.strip_shift);
+      magic_div(g.groups, &g.group_mul, &g.group_shift);
+      magic_div(a.cout, &g.cout_mul, &g.cout_shift);
+      auto go = [&](auto t, auto s, auto v, auto r) {
+        using T = decltype(t);
+        hipLaunchKernelGGL((conv_dw3_strip_kernel<T, decltype(s)::value, decltype(v)::value, decltype(r)::value>),
+                           dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, reinterpret_cast<const T*>(x),
+                           reinterpret_cast<const T*>(w), reinterpret_cast<const T*>(bias), reinterpret_cast<T*>(y), a, g);
+      };
+      auto rows = [&](auto t, auto v) {
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        if (a.sh == 1) { if (R == 1) go(t, I1{}, v, I1{}); else go(t, I1{}, v, I2{}); }
+        else { if (R == 1) go(t, I2{}, v, I1{}); else go(t, I2{}, v, I2{}); }
+      };
+      auto half = [&](auto t) {
+        if (strip == 8) rows(t, std::integral_constant<int, 8>{});
+        else rows(t, std::integral_constant<int, 4>{});
+      };
+      switch (dtype) {
+        case DT_F32: rows(float{}, std::integral_constant<int, 4>{}); break;
+        case DT_F16: half(_Float16{}); break;
+        case DT_BF16: half(__bf16{}); break;
+        default: return hipErrorInvalidValue;
+      }
+      return hipGetLastError();
+    }
+  }
   if (const int rows = dw3_rows(a)) {
     const int64_t blocks = (int64_t)a.N * a.cout * ((a.OH + rows - 1) / rows);
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
