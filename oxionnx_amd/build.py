@@ -20,7 +20,7 @@ LIB = os.path.join(HERE, "libohip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = [f"contract_{dt}_{part}.hip" for dt in ("i8", "f16", "f32", "bf16") for part in ("dense", "conv")] + [ "aux_kernels.hip", "nodes.hip", "ops.cpp", "dispatch.cpp"]
+SOURCES = [f"contract_{dt}_{part}.hip" for dt in ("i8", "f16", "f32", "bf16") for part in ("dense", "conv")] + ["aux_kernels.hip", "skinny.hip", "nodes.hip", "ops.cpp", "dispatch.cpp"]
 
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -35,7 +35,7 @@ def _compile(src, incremental=False):
     if incremental and os.path.exists(obj):
         kern = ["mfma_core.hpp", "launch.hpp", "internal.hpp", "halo_conv.hpp", "norm_stats.hpp"]
         local = {"ops.cpp": ["internal.hpp", "tile_plan.hpp"], "dispatch.cpp": ["internal.hpp"],
-                 "aux_kernels.hip": kern, "nodes.hip": ["internal.hpp", "norm_stats.hpp"]}.get(src, kern + ["contract.inc"])
+                 "aux_kernels.hip": kern, "skinny.hip": kern, "nodes.hip": ["internal.hpp", "norm_stats.hpp"]}.get(src, kern + ["contract.inc"])
         deps = [os.path.join(CSRC, f) for f in [src] + local]
         if src.endswith(".cpp"):
             deps.append(os.path.join(ROOT, "include", "ohip.h"))

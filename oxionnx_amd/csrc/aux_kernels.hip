@@ -101,63 +101,85 @@ template <> struct Vec16<__bf16> {
   }
 };
 
-// One block per weight row n: its 8 waves stride the row's 16-byte chunks
+// One block per NR weight rows: its 8 waves stride the rows' 16-byte chunks
 // together (coalesced, up to 16 loads in flight per lane), reduce through
-// registers and LDS in a fixed order (deterministic), and thread 0 runs the
-// epilogue for the M outputs of that row.
-template <class T, int M>
+// registers and LDS in a fixed order (deterministic), and the first NR * M
+// threads run the epilogue for the outputs of those rows.  Two rows a block
+// share the activation chunks, which the blocks read from L2 (M times the
+// weight's bytes in all with one row a block): 5x4096x4096 f16 23.4 -> 18.9
+// us, 2x4096x1024 f32 6.3 -> 5.2; with fewer weight rows they leave CUs idle
+// (5x25088x512 f16 11.3, 13.0 with two).  Products are summed by fused
+// multiply-adds (that shape 13.4 us with a multiply and an add).
+template <class T, int M, int NR>
 __global__ void __launch_bounds__(512)
-gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, int64_t ldw, int kc,
+gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, int64_t ldw, int kc, int N,
                 FloatEpi<T> epi) {
   constexpr int E = Vec16<T>::N;
   constexpr int kWaves = 8;
-  __shared__ float red[kWaves][M];
-  const int n = blockIdx.x;
+  __shared__ float red[kWaves][NR][M];
+  const int n = blockIdx.x * NR;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const u32x4* wr = reinterpret_cast<const u32x4*>(w + (int64_t)n * ldw);
-  float acc[M];
+  const u32x4* wr[NR];
 #pragma unroll
-  for (int m = 0; m < M; ++m) acc[m] = 0.0f;
-  auto fma_chunk = [&](u32x4 wv, int c) {
-    float f[E];
-    Vec16<T>::unpack(wv, f);
+  for (int i = 0; i < NR; ++i) wr[i] = reinterpret_cast<const u32x4*>(w + (int64_t)min(n + i, N - 1) * ldw);
+  float acc[NR][M];
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const u32x4* ar = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda);
-      float g[E];
-      Vec16<T>::unpack(ar[c], g);
+  for (int i = 0; i < NR; ++i)
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[m] += f[e] * g[e];
-    }
-  };
+    for (int m = 0; m < M; ++m) acc[i][m] = 0.0f;
   constexpr int S = kWaves * 64;
   // loads in flight per lane, issued together (guarded at the row's end):
   // config 2a's K = 25088 row is one round of them in f32 and f16
   // (10.0 -> 9.35 us f32 against four at a time)
-  constexpr int U = sizeof(T) == 4 ? 16 : 8;
+  constexpr int U = (sizeof(T) == 4 ? 16 : 8) / NR;
   for (int c = tid; c < kc; c += U * S) {
-    u32x4 wv[U];
+    u32x4 wv[U][NR];
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (c + u * S < kc) wv[u] = __builtin_nontemporal_load(wr + c + u * S);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c + u * S < kc) fma_chunk(wv[u], c + u * S);
+      for (int i = 0; i < NR; ++i)
+        if (c + u * S < kc) wv[u][i] = __builtin_nontemporal_load(wr[i] + c + u * S);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (c + u * S < kc) {
+        // (all M loads before the first sum: left alone the compiler takes
+        // them one round trip after another)
+        u32x4 av[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) av[m] = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c + u * S];
+        __builtin_amdgcn_sched_barrier(0);
+        float f[NR][E];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) Vec16<T>::unpack(wv[u][i], f[i]);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          float g[E];
+          Vec16<T>::unpack(av[m], g);
+#pragma unroll
+          for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int e = 0; e < E; ++e) acc[i][m] = __builtin_fmaf(f[i][e], g[e], acc[i][m]);
+        }
+      }
+    }
   }
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    float v = acc[m];
+  for (int i = 0; i < NR; ++i)
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) red[wave][m] = v;
-  }
+    for (int m = 0; m < M; ++m) {
+      float v = acc[i][m];
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (lane == 0) red[wave][i][m] = v;
+    }
   __syncthreads();
-  if (tid < M) {
+  if (tid < NR * M && n + tid / M < N) {
+    const int i = tid / M, m = tid - i * M;
     float v = 0.0f;
 #pragma unroll
-    for (int q = 0; q < kWaves; ++q) v += red[q][tid];
+    for (int q = 0; q < kWaves; ++q) v += red[q][i][m];
     // GEMM orientation: i = n (weight row), j = m (activation row)
-    epi.store_one(v, n, tid);
+    epi.store_one(v, n + i, m);
   }
 }
 
@@ -181,14 +203,19 @@ gemv_wave_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, 
 #pragma unroll
   for (int m = 0; m < M; ++m) acc[m] = 0.0f;
   for (int c = lane; c < kc; c += 64) {
+    const u32x4 wv = __builtin_nontemporal_load(wr + c);
+    u32x4 av[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) av[m] = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c];
+    __builtin_amdgcn_sched_barrier(0);   // every load before the first sum, as above
     float f[E];
-    Vec16<T>::unpack(__builtin_nontemporal_load(wr + c), f);
+    Vec16<T>::unpack(wv, f);
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       float g[E];
-      Vec16<T>::unpack(reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c], g);
+      Vec16<T>::unpack(av[m], g);
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[m] += f[e] * g[e];
+      for (int e = 0; e < E; ++e) acc[m] = __builtin_fmaf(f[e], g[e], acc[m]);
     }
   }
 #pragma unroll
@@ -208,6 +235,7 @@ static hipError_t gemv_t(const GemvArgs& g, const FloatOut& o, hipStream_t st) {
   const T* w = reinterpret_cast<const T*>(g.w);
   const FloatEpi<T> epi = make_float_epi<T>(o);
   const bool by_wave = g.kc <= kWaveRowChunks;
+  const int two_rows = sizeof(T) == 4 ? 512 : 1024;   // weight rows from which two a block still fill the chip
   const unsigned wave_blocks = (unsigned)((g.N + 3) / 4);
   switch (g.M) {
 #define OHIP_GEMV_CASE(MM)                                                                                      \
@@ -215,8 +243,11 @@ static hipError_t gemv_t(const GemvArgs& g, const FloatOut& o, hipStream_t st) {
     if (by_wave)                                                                                                \
       hipLaunchKernelGGL((gemv_wave_kernel<T, MM>), dim3(wave_blocks), dim3(256), 0, st, a, g.lda, w, g.ldw, \
                          g.kc, g.N, epi);                                                                       \
+    else if (MM > 1 && g.N >= two_rows)                                                                             \
+      hipLaunchKernelGGL((gemv_row_kernel<T, MM, MM == 1 ? 1 : 2>), dim3((g.N + 1) / 2), dim3(512), 0, st, a, g.lda, w, \
+                         g.ldw, g.kc, g.N, epi);                                                                \
     else                                                                                                        \
-      hipLaunchKernelGGL((gemv_row_kernel<T, MM>), dim3(g.N), dim3(512), 0, st, a, g.lda, w, g.ldw, g.kc, epi); \
+      hipLaunchKernelGGL((gemv_row_kernel<T, MM, 1>), dim3(g.N), dim3(512), 0, st, a, g.lda, w, g.ldw, g.kc, g.N, epi); \
     break;
     OHIP_GEMV_CASE(1) OHIP_GEMV_CASE(2) OHIP_GEMV_CASE(3) OHIP_GEMV_CASE(4)
     OHIP_GEMV_CASE(5) OHIP_GEMV_CASE(6) OHIP_GEMV_CASE(7) OHIP_GEMV_CASE(8)

@@ -23,9 +23,11 @@ inline int forced_splits() {
   return v;
 }
 
-// A block tile and the K slices it runs with (splits > 1: tile 10 or 11).
+// A block tile and the K slices it runs with (splits > 1: tile 10 or 11);
+// us: its estimated time without the launch (0: not estimated).
 struct TilePlan {
   int splits, tile;
+  float us = 0.0f;
 };
 
 // What a block of a tile costs, in us: a stage of 128 bytes of K when its CU
@@ -116,8 +118,10 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   }
   if (best.splits == 1 && kind == PlanKind::Dense && !wide_out) {
     const TileCost& t = kDense[ntab - 1];
-    if (time(t, blocks(t.bp, t.bq), nk) < cost) best.tile = t.id;
+    const float c = time(t, blocks(t.bp, t.bq), nk);
+    if (c < cost) { cost = c; best.tile = t.id; }
   }
+  best.us = cost;
   return best;
 }
 

@@ -1157,3 +1157,59 @@ def test_captured_scratch_outlives_growth(torch):
         assert torch.equal(y, want)
     L.lib().ohip_graph_destroy(g)
     ctx.close()
+
+
+# one and two activation tiles, ragged weight tiles, partial last chunks, rows
+# of any alignment, with and without K slices (5000 x 40)
+@pytest.mark.parametrize("m", [2, 9, 16, 17, 32])
+@pytest.mark.parametrize("k,n", [(1, 5), (7, 16), (64, 33), (777, 130), (5000, 40), (20000, 17)])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_gemm_of_a_few_rows(torch, ctx, m, k, n, dt):
+    from oxionnx_amd import _lib as L
+    rng = np.random.default_rng(m * 31 + k + n)
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    a = _dev(torch, rng.uniform(-1, 1, (m, k + 3)).astype(np.float32)).to(tdt)
+    a[:, :1] = float("nan")   # outside the rows the call reads
+    a[:, k + 1:] = float("inf")
+    b = _dev(torch, rng.normal(0, k ** -0.5, (k, n)).astype(np.float32)).to(tdt)
+    c = _dev(torch, rng.normal(0, 0.1, (m, n)).astype(np.float32)).to(tdt)
+    w = ctx.weight_gemm(b.float().cpu().numpy(), dtype=ldt)
+    rows = a[:, 1:1 + k]
+    y = ctx.gemm(rows, w, c, alpha=0.5, beta=2.0, act=L.ACT_RELU)
+    yt = ctx.gemm(rows.t().contiguous(), w, c, alpha=0.5, beta=2.0, act=L.ACT_RELU, trans_a=True)
+    want = torch.relu(0.5 * (rows.double() @ b.double()) + 2.0 * c.double()).cpu().numpy()
+    for got in (y, yt):
+        assert _rel_err(got.double().cpu().numpy(), want) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+# rows of one and several strips (overlapping at the end), groups of rows cut
+# by the plane, the pads that a strip may reach past, and the geometries
+# beside them (no pad, a pad of two, rows shorter than a run)
+@pytest.mark.parametrize("h,w", [(3, 6), (5, 7), (9, 10), (4, 17), (13, 31), (7, 56), (2, 113), (1, 24), (6, 5), (3, 3)])
+@pytest.mark.parametrize("s,pads", [(1, (1, 1, 1, 1)), (2, (1, 1, 1, 1)), (1, (0, 0, 0, 0)), (2, (0, 0, 1, 1)),
+                                    (1, (2, 2, 2, 2)), (1, (1, 0, 1, 1))], ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_depthwise_3x3_strips(torch, ctx, h, w, s, pads, dt):
+    from oxionnx_amd import _lib as L
+    if h + pads[0] + pads[2] < 3 or w + pads[1] + pads[3] < 3:
+        pytest.skip("the filter does not fit")
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    rng = np.random.default_rng(h * 131 + w)
+    x = _dev(torch, rng.uniform(-1, 1, (2, 5, h, w)).astype(np.float32)).to(tdt)
+    k = _dev(torch, rng.normal(0, 0.3, (5, 1, 3, 3)).astype(np.float32)).to(tdt)
+    k[1, 0, 0, 0] = float("inf")   # a corner tap that only inner outputs have
+    b = _dev(torch, rng.normal(0, 0.1, 5).astype(np.float32)).to(tdt)
+    wt = ctx.weight_conv(k.float().cpu().numpy(), dtype=ldt)
+    y = ctx.conv2d(x, wt, b, strides=(s, s), pads=pads, group=5, act=L.ACT_CLIP, act_lo=-0.5, act_hi=0.5)
+    xp = torch.nn.functional.pad(x.double(), (pads[1], pads[3], pads[0], pads[2]))
+    inside = torch.nn.functional.pad(torch.ones_like(x, dtype=torch.float64), (pads[1], pads[3], pads[0], pads[2]))
+    oh, ow = (xp.shape[2] - 3) // s + 1, (xp.shape[3] - 3) // s + 1
+    want = b.double().reshape(1, 5, 1, 1).expand(2, 5, oh, ow).clone()
+    for ky in range(3):
+        for kx in range(3):
+            at = (slice(None), slice(None), slice(ky, ky + s * (oh - 1) + 1, s), slice(kx, kx + s * (ow - 1) + 1, s))
+            tap = xp[at] * k[:, 0, ky, kx].double().reshape(1, 5, 1, 1)
+            want += torch.where(inside[at] > 0, tap, torch.zeros_like(tap))   # taps outside the image are skipped
+    want = want.clamp(-0.5, 0.5)
+    assert y.shape == want.shape
+    assert torch.allclose(y.double(), want, rtol=0, atol=1e-5 if dt == "f32" else 8e-3, equal_nan=True)
