@@ -223,6 +223,21 @@ def lib():
     return _lib
 
 
+_raw = {}
+
+
+def raw(name):
+    """`name` taking plain integers (addresses), bytes (a packed descriptor) or
+    None for every argument: the form for calls that are made often."""
+    fn = _raw.get(name)
+    if fn is None:
+        fn = lib()[name]   # a function object of its own, beside the typed one
+        fn.restype, args = SIGNATURES[name]
+        fn.argtypes = [VP] * len(args)
+        _raw[name] = fn
+    return fn
+
+
 def last_error():
     return lib().ohip_last_error().decode(errors="replace")
 

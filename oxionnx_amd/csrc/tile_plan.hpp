@@ -92,10 +92,14 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   if (override_tile != 0)
     return {may_split ? (int)std::max<int64_t>(2, std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1)) : 1,
             may_split ? override_tile : override_tile == 11 ? 8 : 9};
-  auto blocks = [&](int bp, int bq) { return (int64_t)((P + bp - 1) / bp) * ((Q + bq - 1) / bq) * batch; };
+  auto blocks = [&](int bp, int bq) {
+    return (int64_t)(((uint32_t)P + (uint32_t)bp - 1) / (uint32_t)bp) * (((uint32_t)Q + (uint32_t)bq - 1) / (uint32_t)bq) *
+           batch;
+  };
   if (nk > 16 && blocks(256, 256) >= 256) return {1, 16};
   auto time = [&](const TileCost& t, int64_t nb, int64_t stages) {
-    const int64_t ncu = (nb + 255) / 256, q = ncu / t.res, rem = ncu % t.res;
+    const uint32_t ncu = (uint32_t)std::min<int64_t>((nb + 255) >> 8, 1 << 24), res = (uint32_t)t.res;
+    const uint32_t q = ncu / res, rem = ncu - q * res;
     return t.fix * (float)(q + (rem ? 1 : 0)) +
            (float)stages * ((float)q * std::max(t.lat, (float)t.res * t.bw) + (rem ? std::max(t.lat, (float)rem * t.bw) : 0.0f));
   };
@@ -105,13 +109,14 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     const TileCost& t = tab[i];
     if (t.id == 18) continue;
     if (wide_out && kind == PlanKind::Dense && t.bp * t.bq > 128 * 128) continue;   // unstaged 4-byte outputs
-    const float c = time(t, blocks(t.bp, t.bq), nk);
+    const int64_t nb = blocks(t.bp, t.bq);
+    const float c = time(t, nb, nk);
     if (c < cost) { cost = c; best = {1, t.id}; }
     if (!may_split || (t.id != 9 && t.id != 8)) continue;
     for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
-      const int64_t per = (nk + s - 1) / s;
+      const uint32_t per = ((uint32_t)nk + s - 1) / s;
       if (per < 2) break;
-      const float cs = time(t, blocks(t.bp, t.bq) * s, per) + red.fix + red.per_slice * (float)s +
+      const float cs = time(t, nb * s, per) + red.fix + red.per_slice * (float)s +
                        red.per_mb * (float)P * (float)Q * (float)batch * (float)s * 4e-6f;
       if (cs < cost) { cost = cs; best = {s, t.id == 9 ? 10 : 11}; }
     }

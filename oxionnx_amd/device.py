@@ -5,29 +5,72 @@ in libohip.so.  The context adopts torch's current stream so library work and
 torch work are ordered without extra synchronisation.
 """
 import ctypes
+import math
+import struct
 
 import numpy as np
 
 from . import _lib as L
 
-_TORCH_DT = None
+# torch.dtype -> element code, and back; filled with the first use of torch
+_OHIP_DT = {}
+_TORCH_DT = {}
 
 
 def _torch():
     import torch
+    if not _OHIP_DT:
+        _TORCH_DT.update({L.F32: torch.float32, L.F16: torch.float16, L.BF16: torch.bfloat16, L.U8: torch.uint8,
+                          L.I8: torch.int8, L.I32: torch.int32})
+        _OHIP_DT.update({t: d for d, t in _TORCH_DT.items()})
     return torch
 
 
 def torch_dtype(dt):
-    torch = _torch()
-    return {L.F32: torch.float32, L.F16: torch.float16, L.BF16: torch.bfloat16, L.U8: torch.uint8,
-            L.I8: torch.int8, L.I32: torch.int32}[dt]
+    _torch()
+    return _TORCH_DT[dt]
 
 
 def ohip_dtype(tdt):
-    torch = _torch()
-    return {torch.float32: L.F32, torch.float16: L.F16, torch.bfloat16: L.BF16, torch.uint8: L.U8,
-            torch.int8: L.I8, torch.int32: L.I32}[tdt]
+    if not _OHIP_DT:
+        _torch()
+    return _OHIP_DT[tdt]
+
+
+class _Packer:
+    """Packs a descriptor of the single-operator calls in C's native layout (its
+    ctypes structure and the pointer objects cost a call more than the launch).
+    Values that only the structure takes (a float beyond f32) go through it."""
+
+    def __init__(self, fmt, desc):
+        self._pack, self._desc = struct.Struct(fmt).pack, desc
+        assert struct.calcsize(fmt) == ctypes.sizeof(desc), "descriptor layout"
+
+    def __call__(self, *values):
+        try:
+            return self._pack(*values)
+        except (struct.error, OverflowError):
+            types = [t for _, t in self._desc._fields_]
+            return bytes(self._desc(*(ctypes.cast(v, t) if issubclass(t, ctypes._Pointer) else v
+                                      for v, t in zip(values, types))))
+
+
+_GEMM = _Packer("@3q2i2f2i2f2q", L.GemmDesc)
+_CONV = _Packer("@16q4i2fi0q", L.ConvDesc)
+_CONVT = _Packer("@18qi0q", L.ConvTDesc)
+_MATMUL = _Packer("@6qi0q", L.MatMulDesc)
+_QGEMM = _Packer("@3qiP2i2f3i2q", L.QGemmDesc)
+# the zero points that one byte can hold, for calls with a single one
+_ZERO_POINTS = np.arange(-128, 256, dtype=np.int32)
+_ZERO_POINTS_AT = _ZERO_POINTS.ctypes.data
+
+
+def _out_dim(size, pad_begin, pad_end, k, dil, stride):
+    """ohip_conv_out_dim."""
+    if stride <= 0 or k <= 0 or dil <= 0 or size < 0 or pad_begin < 0 or pad_end < 0:
+        return -1
+    room = size + pad_begin + pad_end - (k - 1) * dil - 1
+    return -1 if room < 0 else room // stride + 1
 
 
 def _np_ohip_dtype(a):
@@ -36,7 +79,7 @@ def _np_ohip_dtype(a):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _key(name, label):
@@ -195,18 +238,18 @@ class HipContext:
     # --------------------------------------------------------------- ops
     def gemm(self, a, w, c=None, alpha=1.0, beta=1.0, trans_a=False, act=L.ACT_NONE, act_lo=0.0, act_hi=0.0,
              out=None):
-        torch = _torch()
         dt = ohip_dtype(a.dtype)
-        m = a.shape[1] if trans_a else a.shape[0]
+        m = a.size(1) if trans_a else a.size(0)
         k, n = w.shape
         if out is None:
-            out = torch.empty((m, n), dtype=a.dtype, device=a.device)
+            out = _torch().empty((m, n), dtype=a.dtype, device=a.device)
         c_kind = L.C_NONE
         if c is not None:
             c_kind = L.C_SCALAR if c.numel() == 1 else (L.C_ROW if c.dim() == 1 else L.C_FULL)
-        d = L.GemmDesc(m, k, n, dt, int(trans_a), alpha, beta, c_kind, act, act_lo, act_hi,
-                       a.stride(0), out.stride(0))
-        L.check(L.lib().ohip_gemm(self.h, ctypes.byref(d), _ptr(a), w.handle, _ptr(c), _ptr(out)))
+        d = _GEMM(m, k, n, dt, int(trans_a), alpha, beta, c_kind, act, act_lo, act_hi, a.stride(0), out.stride(0))
+        rc = L.raw("ohip_gemm")(self.h, d, a.data_ptr(), w.handle, _ptr(c), out.data_ptr())
+        if rc:
+            L.check(rc)
         return out
 
     def conv2d(self, x, w, bias=None, strides=(1, 1), pads=(0, 0, 0, 0), dilations=(1, 1), act=L.ACT_NONE,
@@ -215,7 +258,6 @@ class HipContext:
         w holds Cin / group input channels per filter (ONNX Conv's group).
         noalloc=True calls ohip_conv2d_noalloc (static scratch, no device
         allocation; `out` should then be given)."""
-        torch = _torch()
         dt = ohip_dtype(x.dtype)
         cout, cin, kh, kw = w.shape
         if in_layout == L.NCHW:
@@ -223,20 +265,23 @@ class HipContext:
         else:
             n, h, wd = x.shape[:3]
             c = cin * group
-        oh = L.lib().ohip_conv_out_dim(h, pads[0], pads[2], kh, dilations[0], strides[0])
-        ow = L.lib().ohip_conv_out_dim(wd, pads[1], pads[3], kw, dilations[1], strides[1])
+        oh = _out_dim(h, pads[0], pads[2], kh, dilations[0], strides[0])
+        ow = _out_dim(wd, pads[1], pads[3], kw, dilations[1], strides[1])
         if oh < 0 or ow < 0:
             raise L.OhipError(L.E_SHAPE, "bad conv geometry")
         if out is None:
+            torch = _torch()
             if out_layout == L.NCHW:
                 out = torch.empty((n, cout, oh, ow), dtype=x.dtype, device=x.device)
             else:
                 ce = 16 // L.ELEM_BYTES[dt]
                 out = torch.zeros((n, oh, ow, (cout + ce - 1) // ce * ce), dtype=x.dtype, device=x.device)
-        d = L.ConvDesc(n, c, h, wd, cout, kh, kw, group, strides[0], strides[1], dilations[0], dilations[1],
-                       pads[0], pads[1], pads[2], pads[3], dt, in_layout, out_layout, act, act_lo, act_hi)
-        fn = L.lib().ohip_conv2d_noalloc if noalloc else L.lib().ohip_conv2d
-        L.check(fn(self.h, ctypes.byref(d), _ptr(x), w.handle, _ptr(bias), _ptr(out)))
+        d = _CONV(n, c, h, wd, cout, kh, kw, group, strides[0], strides[1], dilations[0], dilations[1],
+                       pads[0], pads[1], pads[2], pads[3], dt, in_layout, out_layout, act, act_lo, act_hi, L.PAD_ZEROS)
+        rc = L.raw("ohip_conv2d_noalloc" if noalloc else "ohip_conv2d")(self.h, d, x.data_ptr(), w.handle, _ptr(bias),
+                                                                       out.data_ptr())
+        if rc:
+            L.check(rc)
         return out
 
     def conv2d_instnorm(self, x, w, bias=None, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), eps=1e-5,
@@ -277,23 +322,23 @@ class HipContext:
     def matmul(self, a, b, out=None):
         """Batched MatMul of two device tensors, [..., M, K] x [..., K, N], with the
         reference's slice rule (slice s: A slice s % a_batches, B slice s % b_batches)."""
-        torch = _torch()
         dt = ohip_dtype(a.dtype)
-        batch_shape = list(np.broadcast_shapes(tuple(a.shape[:-2]), tuple(b.shape[:-2])))
-        batch = int(np.prod(batch_shape)) if batch_shape else 1
-        na = int(np.prod(a.shape[:-2])) if a.dim() > 2 else 1
-        nb = int(np.prod(b.shape[:-2])) if b.dim() > 2 else 1
-        m, k, n = a.shape[-2], a.shape[-1], b.shape[-1]
+        sa, sb = tuple(a.shape), tuple(b.shape)
+        m, k, n = sa[-2], sa[-1], sb[-1]
+        na, nb = math.prod(sa[:-2]), math.prod(sb[:-2])
+        batch_shape = sa[:-2] if sa[:-2] == sb[:-2] else np.broadcast_shapes(sa[:-2], sb[:-2])
         if out is None:
-            out = torch.empty(batch_shape + [m, n], dtype=a.dtype, device=a.device)
-        d = L.MatMulDesc(m, k, n, batch, na, nb, dt)
-        L.check(L.lib().ohip_matmul(self.h, ctypes.byref(d), _ptr(a.contiguous()), _ptr(b.contiguous()), _ptr(out)))
+            out = _torch().empty(batch_shape + (m, n), dtype=a.dtype, device=a.device)
+        d = _MATMUL(m, k, n, math.prod(batch_shape), na, nb, dt)
+        a, b = a.contiguous(), b.contiguous()
+        rc = L.raw("ohip_matmul")(self.h, d, a.data_ptr(), b.data_ptr(), out.data_ptr())
+        if rc:
+            L.check(rc)
         return out
 
     def conv_transpose2d(self, x, w, bias=None, strides=(1, 1), pads=(0, 0, 0, 0), dilations=(1, 1),
                          output_padding=(0, 0), group=1, out=None):
         """ConvTranspose, NCHW; pads = [top, left, bottom, right] (already resolved)."""
-        torch = _torch()
         dt = ohip_dtype(x.dtype)
         cin, coutg, kh, kw = w.shape
         n, c, h, wd = x.shape
@@ -302,24 +347,32 @@ class HipContext:
         if oh < 0 or ow < 0:
             raise L.OhipError(L.E_SHAPE, "bad ConvTranspose geometry")
         if out is None:
-            out = torch.empty((n, coutg * group, oh, ow), dtype=x.dtype, device=x.device)
-        d = L.ConvTDesc(n, c, h, wd, coutg * group, kh, kw, group, strides[0], strides[1], dilations[0],
+            out = _torch().empty((n, coutg * group, oh, ow), dtype=x.dtype, device=x.device)
+        d = _CONVT(n, c, h, wd, coutg * group, kh, kw, group, strides[0], strides[1], dilations[0],
                         dilations[1], pads[0], pads[1], pads[2], pads[3], output_padding[0], output_padding[1], dt)
-        L.check(L.lib().ohip_conv_transpose2d(self.h, ctypes.byref(d), _ptr(x), w.handle, _ptr(bias), _ptr(out)))
+        rc = L.raw("ohip_conv_transpose2d")(self.h, d, x.data_ptr(), w.handle, _ptr(bias), out.data_ptr())
+        if rc:
+            L.check(rc)
         return out
 
     def qgemm(self, a, w, a_zp=0, out_kind=L.QOUT_U8, a_scale=1.0, y_scale=1.0, y_zp=0, lo=0, hi=255, out=None):
-        torch = _torch()
         m, k = a.shape
         n = w.shape[1]
-        azp = np.ascontiguousarray(np.atleast_1d(np.asarray(a_zp, np.int32)))
+        if type(a_zp) is int and -128 <= a_zp <= 255:
+            azp_at, n_azp = _ZERO_POINTS_AT + 4 * (a_zp + 128), 1
+        else:
+            azp = np.ascontiguousarray(np.atleast_1d(np.asarray(a_zp, np.int32)))
+            azp_at, n_azp = azp.ctypes.data, azp.size
         if out is None:
+            torch = _torch()
             odt = {L.QOUT_U8: torch.uint8, L.QOUT_I8: torch.int8, L.QOUT_I32: torch.int32,
                    L.QOUT_F32: torch.float32}[out_kind]
             out = torch.empty((m, n), dtype=odt, device=a.device)
-        d = L.QGemmDesc(m, k, n, ohip_dtype(a.dtype), azp.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
-                        azp.size, out_kind, a_scale, y_scale, y_zp, lo, hi, a.stride(0), out.stride(0))
-        L.check(L.lib().ohip_qgemm(self.h, ctypes.byref(d), _ptr(a), w.handle, _ptr(out)))
+        d = _QGEMM(m, k, n, ohip_dtype(a.dtype), azp_at, n_azp, out_kind, a_scale, y_scale, y_zp, lo, hi,
+                        a.stride(0), out.stride(0))
+        rc = L.raw("ohip_qgemm")(self.h, d, a.data_ptr(), w.handle, out.data_ptr())
+        if rc:
+            L.check(rc)
         return out
 
     def qconv2d(self, x, w, bias=None, x_zp=0, out_kind=L.QOUT_U8, x_scale=1.0, y_scale=1.0, y_zp=0, lo=0,
