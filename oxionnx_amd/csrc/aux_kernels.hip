@@ -1010,8 +1010,14 @@ hipError_t run_conv_fewco(int dtype, const void* x, int pitch, const void* w, co
 // tap from the patch at pixel offset kx: no NHWC staging transpose, and the
 // input is fetched once per slab instead of once per tap.  A block is one
 // 64-pixel segment of an output row x 64 output channels, four waves of
-// 32 x 32; the next slab's loads are issued into registers before the
-// current slab's MFMAs and stored after them (two LDS buffers).  k runs
+// 32 x 32; the loads of the slab after the next are issued into registers
+// before the current slab's MFMAs, and the next slab's are stored after them
+// (two LDS buffers, two register sets: a slab's 36 MFMAs are 1 us, less than
+// a load's round trip; 1x64x128x128 -> 64 21.0 -> 18.9 us, 20.7 with one set).
+// A block a CU and one wave a SIMD leave the LDS reads before each MFMA
+// exposed: 64 TFLOP/s there, 41 % of the f32 rate.  The loads go through buffer resources from per-thread
+// offsets formed once; elements outside the image, the channels or the filter
+// read zero through the range check, so the loop has no branch.  k runs
 // (tap, channel): MFMA step j covers k = 2j, 2j + 1, one tap and channels
 // 2j % 8 + {0, 1}, so both operands' addresses are a per-lane base plus a
 // compile-time offset.
@@ -1037,48 +1043,63 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
   const float* xn = x + (int64_t)n * a.C * a.H * a.W;
   const int slabs = (a.C + kF32Cs - 1) / kF32Cs;
 
-  float pv[NP];
-  f32x4 fv[NF];
-  auto load = [&](int sl) __attribute__((always_inline)) {
-    const int c0 = sl * kF32Cs;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xn, (short)0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rf =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)co0 * a.ldw), (short)0, 0x7fffffff, 0x00020000);
+  // this thread's patch elements and filter chunks of a slab: byte offsets at
+  // slab 0 and the channel (of a chunk: its first) within the slab
+  int poff[NP], pc[NP], foff[NF], fc[NF];
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
-      const int i = t + u * 256;
-      const int px = i % PWP, r = i / PWP, ky = r % KH, c = r / KH;
-      int iy = oy + ky, ix = ox0 + px;   // padded coordinates
-      bool ok = i < PATCH && c0 + c < a.C;
-      if constexpr (!MAPPED) {
-        iy -= a.pt;
-        ix -= a.pl;
-        ok = ok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-      } else {
-        iy = pad_map(iy, a.pt, a.H, a.pad_mode);
-        ix = pad_map(ix, a.pl, a.W, a.pad_mode);
-      }
-      pv[u] = ok ? xn[((int64_t)(c0 + c) * a.H + iy) * a.W + ix] : 0.0f;
+  for (int u = 0; u < NP; ++u) {
+    const int i = t + u * 256;
+    const int px = i % PWP, r = i / PWP, ky = r % KH, c = r / KH;
+    int iy = oy + ky, ix = ox0 + px;   // padded coordinates
+    bool ok = i < PATCH;
+    if constexpr (!MAPPED) {
+      iy -= a.pt;
+      ix -= a.pl;
+      ok = ok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+    } else {
+      iy = pad_map(iy, a.pt, a.H, a.pad_mode);
+      ix = pad_map(ix, a.pl, a.W, a.pad_mode);
     }
+    pc[u] = c;
+    poff[u] = ok ? (int)((((int64_t)c * a.H + iy) * a.W + ix) * 4) : kOobOffset;
+  }
 #pragma unroll
-    for (int u = 0; u < NF; ++u) {
-      const int i = t + u * 256;        // (co, tap, half)
-      const int h = i & 1, r = i >> 1, tap = r % TAPS, co = r / TAPS;
-      const bool ok = i < kF32Co * TAPS * 2 && co0 + co < a.cout && c0 + 4 * h < a.cpg;
-      fv[u] = ok ? *reinterpret_cast<const f32x4*>(w + (int64_t)(co0 + co) * a.ldw + (int64_t)tap * a.cpg + c0 + 4 * h)
-                 : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+  for (int u = 0; u < NF; ++u) {
+    const int i = t + u * 256;        // (co, tap, half)
+    const int h = i & 1, r = i >> 1, tap = r % TAPS, co = r / TAPS;
+    fc[u] = 4 * h;
+    foff[u] = i < kF32Co * TAPS * 2 && co0 + co < a.cout ? (int)(((int64_t)co * a.ldw + (int64_t)tap * a.cpg + 4 * h) * 4)
+                                                         : kOobOffset;
+  }
+  struct Slab { float p[NP]; u32x4 f[NF]; };
+  auto load = [&](Slab& d, int sl) __attribute__((always_inline)) {
+    const int c0 = sl * kF32Cs, left = a.C - c0, leftf = a.cpg - c0;   // (<= 0 past the last slab: all read zero)
+    const int so = __builtin_amdgcn_readfirstlane(left > 0 ? (int)((int64_t)c0 * a.H * a.W * 4) : 0);
+    const int sf = __builtin_amdgcn_readfirstlane(leftf > 0 ? c0 * 4 : 0);
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      d.p[u] = lane_f32((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rx, pc[u] < left ? poff[u] : kOobOffset, so, 0));
+#pragma unroll
+    for (int u = 0; u < NF; ++u)
+      d.f[u] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rf, fc[u] < leftf ? foff[u] : kOobOffset, sf, 0));
   };
-  auto store = [&](int b) __attribute__((always_inline)) {
+  auto store = [&](const Slab& s, int b) __attribute__((always_inline)) {
     float* pd = lds[b];
     float* fd = lds[b] + PATCH;
 #pragma unroll
     for (int u = 0; u < NP; ++u)
-      if (t + u * 256 < PATCH) pd[t + u * 256] = pv[u];
+      if (t + u * 256 < PATCH) pd[t + u * 256] = s.p[u];
 #pragma unroll
     for (int u = 0; u < NF; ++u) {
       const int i = t + u * 256;
       if (i < kF32Co * TAPS * 2) {
         const int h = i & 1, r = i >> 1, tap = r % TAPS, co = r / TAPS;
         float* d = fd + co * FST + tap * kF32Cs + 4 * h;
-        d[0] = fv[u][0]; d[1] = fv[u][1]; d[2] = fv[u][2]; d[3] = fv[u][3];
+        d[0] = lane_f32(s.f[u].x); d[1] = lane_f32(s.f[u].y); d[2] = lane_f32(s.f[u].z); d[3] = lane_f32(s.f[u].w);
       }
     }
   };
@@ -1088,12 +1109,16 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
   for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
   const int abase = kk * KH * PWP + wp * 32 + m;   // channel kk of the pair, this lane's pixel
   const int bbase = (wq * 32 + m) * FST + kk;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int sl = 0; sl < slabs; ++sl) {
+  // a wave whose pixels or channels all lie past the output's edge only stages
+  const bool busy = ox0 + __builtin_amdgcn_readfirstlane(wp) * 32 < a.OW &&
+                    co0 + __builtin_amdgcn_readfirstlane(wq) * 32 < a.cout;
+  // one slab: `next` holds the loads of slab sl + 1, `after` takes those of
+  // sl + 2
+  auto step = [&](int sl, const Slab& next, Slab& after) __attribute__((always_inline)) {
     const int b = sl & 1;
-    if (sl + 1 < slabs) load(sl + 1);
+    load(after, sl + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    if (busy) {
     const float* pa = lds[b] + abase;
     const float* pb = lds[b] + PATCH + bbase;
 #pragma unroll
@@ -1104,9 +1129,25 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
       const float bv = pb[2 * j];
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
     }
-    if (sl + 1 < slabs) store(b ^ 1);
-    __syncthreads();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    store(next, b ^ 1);   // (past the last slab: zeros that nobody reads)
+    // (no __syncthreads: its fence would drain the loads in flight)
+    wait_lgkm0();
+    barrier_only();
+  };
+  Slab s0, s1;
+  load(s0, 0);
+  load(s1, 1);
+  store(s0, 0);
+  wait_lgkm0();
+  barrier_only();
+  int sl = 0;
+  for (; sl + 1 < slabs; sl += 2) {   // (pairs without a condition: the waits stay counts)
+    step(sl, s1, s0);
+    step(sl + 1, s0, s1);
   }
+  if (sl < slabs) step(sl, s1, s0);
   // lane: pixels wp * 32 + 8g + 4kk + e, output channel wq * 32 + m
   const int co = co0 + wq * 32 + m;
   if (co >= a.cout) return;
@@ -1130,7 +1171,9 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
 
 bool conv_nchw_f32_supported(const DirectConvArgs& a) {
   return a.KH == a.KW && (a.KH == 3 || (a.KH == 1 && a.pad_mode == 0)) && a.sh == 1 && a.sw == 1 && a.dh == 1 && a.dw == 1 &&
-         !a.nhwc_out && a.cpg % 4 == 0 && a.ldw % 4 == 0;
+         !a.nhwc_out && a.cpg % 4 == 0 && a.ldw % 4 == 0 &&
+         // 32-bit buffer offsets
+         ((int64_t)a.C + kF32Cs) * a.H * a.W * 4 < 0x7fffffff && (int64_t)kF32Co * a.ldw * 4 < 0x7fffffff;
 }
 
 hipError_t run_conv_nchw_f32(const float* x, const float* w, const float* bias, float* y, const DirectConvArgs& a,

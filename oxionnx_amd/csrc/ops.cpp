@@ -1403,6 +1403,29 @@ struct ConvNorm {
 // plane): nothing has been launched, and the caller runs the two steps.
 constexpr int kNormTwoStep = 1 << 20;
 
+// Whether an f32 convolution that conv_nchw_f32_kernel could read in place is
+// faster staged on the engine, by estimated times in us (fitted to 18 shapes
+// of 8-160 pixels, 20-256 channels, graph replay).  The in-place kernel's
+// blocks are whole 64-pixel row segments x 64 channels, a slab of eight
+// channels at a time: ragged rows, few channels and a second round of blocks
+// cost it whole blocks, where the engine tiles the flattened pixels and may
+// split K (4x256x14x14 -> 256 3x3: 25.8 against 52.7 us, 4x96x72x72 -> 96: 60
+// against 89, 6x48x58x65 -> 144: 58 against 97; 1x64x128x128 -> 64 stays in
+// place: 18.9 against 25.6).
+static bool staged_f32_wins(ohip_ctx* ctx, const ohip_conv_desc* d, int64_t rows, const ConvGeo& g, int64_t cp,
+                            size_t staged, bool noalloc) {
+  if (ctx->tile_override != 0 || forced_splits()) return false;
+  const bool k3 = d->kh == 3;
+  const TilePlan sc = plan_tiles(PlanKind::DenseF32, (int)rows, (int)d->cout, (int)(d->kh * d->kw * (cp / 4)), 0);
+  // its scratch has to fit an allocation-free call
+  if (noalloc && staged + split_ws_bytes((int)rows, (int)d->cout, sc.splits) + 512 > kStaticScratchBytes) return false;
+  const float blocks = (float)(d->n * g.oh * ((g.ow + 63) / 64) * ((d->cout + 63) / 64)) * (g.ow <= 32 ? 0.55f : 1.0f);
+  const float n = std::ceil(blocks / 256.0f), slabs = (float)((d->c + 7) / 8);
+  const float in_place = 3.3f + slabs * (n <= 1.0f ? (k3 ? 1.75f : .31f) : n * (k3 ? 1.65f : .33f));
+  const float staging = 2.6f + (float)staged * 2e-6f / 2.5f;
+  return 1.15f * (sc.us + 3.1f + staging) < in_place;
+}
+
 static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohip_weight* w, const void* bias,
                        void* y, bool noalloc, const ConvNorm* norm = nullptr) {
   int rc = activate(ctx);
@@ -1512,7 +1535,8 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
       (fused_pad ? (d->h + d->pad_t + d->pad_b) * (d->w + d->pad_l + d->pad_r) : d->h * d->w) * cpt * eb;
   if (!norm && !direct && !fewout && d->dtype == OHIP_F32 && G == 1 && d->in_layout == OHIP_NCHW &&
       nchw_f32_allowed() && conv_nchw_f32_supported(a) && !wk_plan(ctx, d, G, staged_w, g, staged_bytes) &&
-      halo_plan(ctx, d, G, staged_w, g, (int)(cp / ce), staged_bytes) == 0) {
+      halo_plan(ctx, d, G, staged_w, g, (int)(cp / ce), staged_bytes) == 0 &&
+      !staged_f32_wins(ctx, d, rows, g, cp, (size_t)(d->n * staged_bytes), noalloc)) {
     ctx->counters.contraction_launches++;
     hipError_t e = run_conv_nchw_f32(static_cast<const float*>(x), static_cast<const float*>(w->data),
                                      static_cast<const float*>(bias), static_cast<float*>(y), a, ctx->stream);
