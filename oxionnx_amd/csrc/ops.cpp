@@ -201,6 +201,19 @@ static int scratch_reserve(ohip_ctx* ctx, size_t bytes) {
   return OHIP_OK;
 }
 
+// Whether `bytes` of scratch cannot be had now because the context's stream is
+// capturing (growing waits for the stream and allocates): a call that can do
+// without, by running unsplit or in place, then does.
+static bool scratch_frozen(ohip_ctx* ctx, size_t bytes) {
+  if (bytes <= ctx->scratch_bytes) return false;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status == hipStreamCaptureStatusActive;
+}
+
 static void* scratch_at(ohip_ctx* ctx, const ScratchPlan& p, size_t idx) {
   size_t off = 0;
   for (size_t i = 0; i < idx; ++i) off += p.sizes[i];
@@ -1216,6 +1229,8 @@ extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, 
                       skinny_wins(d->dtype, M, N, b->kc, packed && !d->trans_a, sc.us);
   const bool gemv = M <= kMaxGemvM && !skinny;
   if (skinny) sc = TilePlan{1, 0};
+  if (sc.splits > 1 && scratch_frozen(ctx, split_ws_bytes((int)N, (int)M, sc.splits) + 256))
+    sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, b->kc, ctx->tile_override, 1, false, false);
   const bool direct = !packed || (skinny && !d->trans_a);
 
   ScratchPlan plan;
@@ -1417,8 +1432,9 @@ static bool staged_f32_wins(ohip_ctx* ctx, const ohip_conv_desc* d, int64_t rows
   if (ctx->tile_override != 0 || forced_splits()) return false;
   const bool k3 = d->kh == 3;
   const TilePlan sc = plan_tiles(PlanKind::DenseF32, (int)rows, (int)d->cout, (int)(d->kh * d->kw * (cp / 4)), 0);
-  // its scratch has to fit an allocation-free call
-  if (noalloc && staged + split_ws_bytes((int)rows, (int)d->cout, sc.splits) + 512 > kStaticScratchBytes) return false;
+  // its scratch has to fit an allocation-free call, and be there under capture
+  const size_t need = staged + split_ws_bytes((int)rows, (int)d->cout, sc.splits) + 512;
+  if (noalloc ? need > kStaticScratchBytes : scratch_frozen(ctx, need)) return false;
   const float blocks = (float)(d->n * g.oh * ((g.ow + 63) / 64) * ((d->cout + 63) / 64)) * (g.ow <= 32 ? 0.55f : 1.0f);
   const float n = std::ceil(blocks / 256.0f), slabs = (float)((d->c + 7) / 8);
   const float in_place = 3.3f + slabs * (n <= 1.0f ? (k3 ? 1.75f : .31f) : n * (k3 ? 1.65f : .33f));
@@ -1527,7 +1543,7 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   // f32 3x3 / 1x1 stride-1 convolutions of an NCHW input, NCHW out: the
   // patch-staged kernel reads the input as it is, a fused reflect / edge pad
   // included (no staging transpose;
-  // config 1: 27.7 -> 20.9 us).  Long reductions over few pixels keep the
+  // 1x64x128x128 -> 64: 27.7 -> 18.9 us).  Long reductions over few pixels keep the
   // halo-patch path, whose split-K fills the chip, and so do the ones the
   // whole-K kernel takes (the sums a fused norm's conv makes, bit for bit).
   const int64_t staged_w = fused_pad ? d->w + d->pad_l + d->pad_r : d->w;
@@ -1584,10 +1600,12 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
                 : hsplits ? TilePlan{hsplits, 0}
                           : plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override,
                                        (int)G);
-  // a static scratch too small for the slices' partial sums: no split
-  if (noalloc && !wk && !hsplits && sc.splits > 1 &&
-      split_ws_bytes(sP, sQ, sc.splits) * (size_t)G + (stage ? (size_t)(d->n * sh_ * sw_ * cpt) * eb : 0) + 512 >
-          kStaticScratchBytes)
+  // a static scratch too small for the slices' partial sums, or one that
+  // cannot grow under capture: no split
+  const size_t sneed =
+      split_ws_bytes(sP, sQ, sc.splits) * (size_t)G + (stage ? (size_t)(d->n * sh_ * sw_ * cpt) * eb : 0) + 512;
+  if (!wk && !hsplits && sc.splits > 1 &&
+      (noalloc ? sneed > kStaticScratchBytes : !norm && scratch_frozen(ctx, sneed)))
     sc = plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override, (int)G, false, false);
   const int splits = sc.splits;
   if (norm && splits == 1 && !wk) {   // counted again by the two-step path's plain call
@@ -1861,8 +1879,11 @@ extern "C" int ohip_matmul(ohip_ctx* ctx, const ohip_matmul_desc* d, const void*
   ScratchPlan plan;
   size_t ib = plan.add((size_t)(d->b_batches * N * kp) * eb);
   size_t ia = a_direct ? SIZE_MAX : plan.add((size_t)(d->a_batches * M * kp) * eb);
-  const TilePlan sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce),
-                                 plain_tile_id(ctx->tile_override) ? ctx->tile_override : 0, (int)d->batch);
+  const int forced = plain_tile_id(ctx->tile_override) ? ctx->tile_override : 0;
+  TilePlan sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce), forced, (int)d->batch);
+  if (sc.splits > 1 &&
+      scratch_frozen(ctx, plan.total() + split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch + 256))
+    sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce), forced, (int)d->batch, false, false);
   size_t iw = sc.splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
   if (rc) return rc;
@@ -2070,7 +2091,9 @@ extern "C" int ohip_qgemm(ohip_ctx* ctx, const ohip_qgemm_desc* d, const void* a
   size_t ia = direct ? SIZE_MAX : plan.add((size_t)(M * kp));
   size_t ir = d->n_azp > 1 ? plan.add((size_t)M * 4) : SIZE_MAX;
   const int ob = (d->out_kind == OHIP_QOUT_I32 || d->out_kind == OHIP_QOUT_F32) ? 4 : 1;
-  const TilePlan sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4);
+  TilePlan sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4);
+  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + split_ws_bytes((int)N, (int)M, sc.splits) + 256))
+    sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4, false);
   const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, splits)) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
@@ -2199,7 +2222,9 @@ extern "C" int ohip_qconv2d(ohip_ctx* ctx, const ohip_qconv_desc* d, const void*
   const bool stage = d->in_layout == OHIP_NCHW;
   size_t ix = stage ? plan.add((size_t)(d->n * d->h * d->w * cpt)) : SIZE_MAX;
   const int sP = nchw_out ? (int)rows : (int)coutg, sQ = nchw_out ? (int)coutg : (int)rows;
-  const TilePlan sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4);
+  TilePlan sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4);
+  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + split_ws_bytes(sP, sQ, sc.splits) + 256))
+    sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4, false);
   const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes(sP, sQ, splits)) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());

@@ -1159,6 +1159,53 @@ def test_captured_scratch_outlives_growth(torch):
     ctx.close()
 
 
+@pytest.mark.parametrize("op", ["gemm", "conv", "qgemm"])
+def test_capture_without_scratch(torch, op):
+    """A call that needs scratch only for its K slices or its staging is
+    captured on a context that has none: unsplit, or in place."""
+    import ctypes
+
+    from oxionnx_amd import _lib as L
+    from oxionnx_amd.device import HipContext
+    ctx = HipContext(0)
+    rng = np.random.default_rng(5)
+    if op == "conv":
+        x = _dev(torch, rng.integers(-3, 4, (4, 128, 14, 14)).astype(np.float32))
+        w = ctx.weight_conv(rng.integers(-3, 4, (64, 128, 3, 3)).astype(np.float32), dtype=L.F32)
+        y = torch.empty((4, 64, 14, 14), dtype=torch.float32, device="cuda")
+        call = lambda: ctx.conv2d(x, w, pads=(1, 1, 1, 1), out=y)
+    elif op == "gemm":
+        x = _dev(torch, rng.integers(-3, 4, (64, 4096)).astype(np.float32)).half()
+        w = ctx.weight_gemm(rng.integers(-3, 4, (4096, 64)).astype(np.float32), dtype=L.F16)
+        y = torch.empty((64, 64), dtype=torch.float16, device="cuda")
+        call = lambda: ctx.gemm(x, w, out=y)
+    else:
+        x = _dev(torch, rng.integers(0, 256, (64, 4096)).astype(np.uint8))
+        w = ctx.weight_qgemm(rng.integers(-128, 128, (4096, 64)).astype(np.int8), zp=0)
+        y = torch.empty((64, 64), dtype=torch.int32, device="cuda")
+        call = lambda: ctx.qgemm(x, w, a_zp=3, out_kind=L.QOUT_I32, out=y)
+    torch.cuda.synchronize()
+    g = ctypes.c_void_p()
+    allocs = ctx.counters()["device_allocs"]
+    L.check(L.lib().ohip_graph_begin(ctx.h))
+    call()
+    L.check(L.lib().ohip_graph_end(ctx.h, ctypes.byref(g)))
+    assert ctx.counters()["device_allocs"] == allocs
+    got = []
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        L.check(L.lib().ohip_graph_launch(g))
+        ctx.sync()
+        got.append(y.clone())
+    call()   # eager: the slices, or the staging, in scratch (whole numbers: the same sums in any order)
+    ctx.sync()
+    assert ctx.counters()["device_allocs"] > allocs
+    assert all(torch.equal(v, y) for v in got)
+    L.lib().ohip_graph_destroy(g)
+    ctx.close()
+
+
 # one and two activation tiles, ragged weight tiles, partial last chunks, rows
 # of any alignment, with and without K slices (5000 x 40)
 @pytest.mark.parametrize("m", [2, 9, 16, 17, 32])
