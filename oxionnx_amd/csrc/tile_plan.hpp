@@ -56,6 +56,10 @@ enum class PlanKind { Dense, DenseF32, Conv };   // f16 / bf16 / int8 rows; f32 
 // Grids of a round of 256x256 tiles and a long K take tile 16 outright: its
 // advantage there is the clock and the cache, which the stages' cost does
 // not show (4096x4096x11008 f16 291 us against 324 on tiles 3, 4 and 18).
+// A convolution's tile 1 is charged 0.5 us a round above its fit: the fit's
+// replays find every operand in the cache, a forward's convolution does not,
+// and two LDS stages hide less of that than tile 9's four (512 blocks of a
+// generator's 3x3 stride-2 f16 convolution 11.7 us on tile 1, 10.4 on 9).
 // The split is symmetric in P and Q (a convolution splits alike in NCHW and
 // NHWC output), so it is chosen without the one tile that is not square or
 // paired, 18 (whose 4-byte outputs do not fit its stage buffers: wide_out).
@@ -70,7 +74,7 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
                                       {8, 128, 128, 2, 1.80f, 1.92f, 1.65f},  {12, 128, 128, 1, 2.04f, 2.04f, 1.68f},
                                       {3, 256, 128, 1, 3.47f, 3.47f, 2.25f},  {4, 128, 256, 1, 3.47f, 3.47f, 2.25f},
                                       {16, 256, 256, 1, 7.09f, 7.09f, 7.69f}};
-  static constexpr TileCost kConv[] = {{1, 64, 64, 4, .522f, .234f, .67f},    {9, 64, 64, 2, .386f, .254f, 1.17f},
+  static constexpr TileCost kConv[] = {{1, 64, 64, 4, .522f, .234f, 1.17f},   {9, 64, 64, 2, .386f, .254f, 1.17f},
                                        {8, 128, 128, 2, .633f, .403f, 1.56f}, {12, 128, 128, 1, .510f, .510f, 2.15f},
                                        {3, 256, 128, 1, .708f, .708f, 4.0f},  {4, 128, 256, 1, .708f, .708f, 4.0f}};
   // (+ 1.5: a launch more also costs the host about 2 us, which small eager
