@@ -111,7 +111,7 @@ template <> struct Vec16<__bf16> {
 // (5x25088x512 f16 11.3, 13.0 with two).  Products are summed by fused
 // multiply-adds (that shape 13.4 us with a multiply and an add).
 template <class T, int M, int NR>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, sizeof(T) == 2 && NR == 1 ? 6 : 1)
 gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, int64_t ldw, int kc, int N,
                 FloatEpi<T> epi) {
   constexpr int E = Vec16<T>::N;
@@ -132,6 +132,11 @@ gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, i
   // config 2a's K = 25088 row is one round of them in f32 and f16
   // (10.0 -> 9.35 us f32 against four at a time)
   constexpr int U = (sizeof(T) == 4 ? 16 : 8) / NR;
+  // activation loads issued together: all M, or half of them where all would
+  // leave a CU two blocks instead of three (8x5952x640 bf16 10.4 -> 9.0 us,
+  // 7x5952x640 f16 10.3 -> 8.1; with three anyway they lose 1-6 %)
+  constexpr bool half = sizeof(T) == 2 && NR == 1 && M >= (std::is_same<T, __bf16>::value ? 6 : 7);
+  constexpr int AB = half ? (M + 1) / 2 : M;
   for (int c = tid; c < kc; c += U * S) {
     u32x4 wv[U][NR];
 #pragma unroll
@@ -142,23 +147,28 @@ gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, i
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (c + u * S < kc) {
-        // (all M loads before the first sum: left alone the compiler takes
-        // them one round trip after another)
-        u32x4 av[M];
-#pragma unroll
-        for (int m = 0; m < M; ++m) av[m] = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c + u * S];
-        __builtin_amdgcn_sched_barrier(0);
+        // (up to AB loads before their first sum: left alone the compiler
+        // takes them one round trip after another)
         float f[NR][E];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) Vec16<T>::unpack(wv[u][i], f[i]);
+        for (int m0 = 0; m0 < M; m0 += AB) {
+          u32x4 av[AB];
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-          float g[E];
-          Vec16<T>::unpack(av[m], g);
+          for (int m = m0; m < m0 + AB && m < M; ++m)
+            av[m - m0] = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c + u * S];
+          __builtin_amdgcn_sched_barrier(0);
+          if (m0 == 0)
 #pragma unroll
-          for (int i = 0; i < NR; ++i)
+            for (int i = 0; i < NR; ++i) Vec16<T>::unpack(wv[u][i], f[i]);
 #pragma unroll
-            for (int e = 0; e < E; ++e) acc[i][m] = __builtin_fmaf(f[i][e], g[e], acc[i][m]);
+          for (int m = m0; m < m0 + AB && m < M; ++m) {
+            float g[E];
+            Vec16<T>::unpack(av[m - m0], g);
+#pragma unroll
+            for (int i = 0; i < NR; ++i)
+#pragma unroll
+              for (int e = 0; e < E; ++e) acc[i][m] = __builtin_fmaf(f[i][e], g[e], acc[i][m]);
+          }
         }
       }
     }
@@ -235,7 +245,11 @@ static hipError_t gemv_t(const GemvArgs& g, const FloatOut& o, hipStream_t st) {
   const T* w = reinterpret_cast<const T*>(g.w);
   const FloatEpi<T> epi = make_float_epi<T>(o);
   const bool by_wave = g.kc <= kWaveRowChunks;
-  const int two_rows = sizeof(T) == 4 ? 512 : 1024;   // weight rows from which two a block still fill the chip
+  // weight rows from which two a block still fill the chip; earlier where the
+  // registers leave a CU three blocks of one row each and those need a second
+  // round (3x5000x1000 bf16 7.7 -> 6.0 us, 6x5200x900 9.6 -> 8.3)
+  const int m3 = std::is_same<T, __bf16>::value ? 3 : 5;
+  const int two_rows = sizeof(T) == 4 ? 512 : g.M >= m3 ? 769 : 1024;
   const unsigned wave_blocks = (unsigned)((g.N + 3) / 4);
   switch (g.M) {
 #define OHIP_GEMV_CASE(MM)                                                                                      \
@@ -1465,7 +1479,7 @@ inline int dw3_strip(const DirectConvArgs& a, int elem_bytes) {
 // at most about eight outputs a thread, within the window's LDS budget;
 // 0 when the geometry is not its.
 inline int dw3_rows(const DirectConvArgs& a) {
-  // OHIP_DW3=0 keeps these convolutions on conv_direct_kernel (a measurement switch)
+  // OHIP_DW3=0 keeps them on conv_direct_kernel (a measurement switch)
   static const bool on = [] { const char* e = std::getenv("OHIP_DW3"); return !(e && e[0] == '0'); }();
   if (!on) return 0;
   if (!(a.cg == 1 && a.coutg == 1 && a.KH == 3 && a.KW == 3 && a.dh == 1 && a.dw == 1 && a.sh == a.sw &&
