@@ -77,8 +77,9 @@ int ohip_sync(ohip_ctx* ctx);
  * Capture of a whole forward into one HIP graph (the reference's CUDA-graph
  * cache, oxionnx-cuda/src/graph_cache.rs): ohip_graph_begin opens a capture
  * on the context's stream; every dispatch until ohip_graph_end is recorded,
- * not run.  Dispatches must already be warm (weights, constants and output
- * tables cached), because uploads and synchronisations cannot be captured.
+ * not run.  Dispatches must already be warm (weights, constants, scratch and
+ * output tables), because uploads, allocations and synchronisations cannot be
+ * captured; a call that can do without missing scratch (unsplit) does.
  * While a capture is open, freed device buffers are parked for the graph,
  * which keeps them until ohip_graph_destroy; a replay writes the same
  * buffers, so the caller keeps the captured inputs and outputs alive and
@@ -202,8 +203,8 @@ typedef struct {
 int ohip_matmul(ohip_ctx* ctx, const ohip_matmul_desc* d, const void* a, const void* b, void* y);
 
 /* Conv, rank 2, any group (oxionnx-ops/src/registry/conv_ops/conv.rs:163-323
- * and conv_typed.rs:54-153): Y = act(conv(X, W) + bias).  Groups run one
- * MFMA launch each, or a direct kernel when a group is too narrow for an
+ * and conv_typed.rs:54-153): Y = act(conv(X, W) + bias).  Groups run
+ * in one MFMA launch, or a direct kernel when a group is too narrow for an
  * MFMA tile (depthwise).  Pads are
  * [top, left, bottom, right], already resolved from auto_pad
  * (conv/spatial.rs:228-257); asymmetric pads are supported.  NCHW inputs are
@@ -231,8 +232,9 @@ int ohip_conv2d(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohi
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * kernels and results as ohip_conv2d; the NCHW staging copy and the split-K
  * partial sums live in a static 32 MiB device array per GPU instead of the
- * context's growable scratch.  A call needing more scratch than that returns
- * OHIP_E_NOMEM and launches nothing.  Every call on one GPU shares the array,
+ * context's growable scratch.  A call that fits there only unsplit, or only
+ * unstaged, runs so; one needing more scratch still returns OHIP_E_NOMEM and
+ * launches nothing.  Every call on one GPU shares the array,
  * so calls that overlap on one GPU (other streams or contexts) race. */
 int ohip_conv2d_noalloc(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohip_weight* w,
                         const void* bias, void* y);

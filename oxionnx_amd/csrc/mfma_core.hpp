@@ -413,8 +413,8 @@ struct OutAddr {
   }
   // bytes from slice 0's output to that of slice blockIdx.z
   __device__ __forceinline__ int64_t slice_offset() const {
-    if (batch <= 1) return 0;
     const int z = (int)blockIdx.z;
+    if (z == 0 || batch <= 1) return 0;
     return zsw > 0 ? (int64_t)(z / zsw) * zrow + (int64_t)(z % zsw) * zstride : (int64_t)z * zstride;
   }
 };
@@ -692,7 +692,7 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
     }
   };
   auto flush_any = [&](auto ebc) __attribute__((always_inline)) {
-    if (!ragged) flush(ebc);
+    if (__builtin_expect(!ragged, 1)) flush(ebc);   // (the common path stays contiguous)
     else if (out.vec) flush_ragged(ebc, std::integral_constant<int, 4>{});
     else flush_ragged(ebc, std::integral_constant<int, 1>{});
   };
