@@ -214,7 +214,9 @@ static bool scratch_frozen(ohip_ctx* ctx, size_t bytes) {
   return status == hipStreamCaptureStatusActive;
 }
 
+// (null when nothing was ever reserved: a plan of no bytes)
 static void* scratch_at(ohip_ctx* ctx, const ScratchPlan& p, size_t idx) {
+  if (!ctx->scratch) return nullptr;
   size_t off = 0;
   for (size_t i = 0; i < idx; ++i) off += p.sizes[i];
   return static_cast<char*>(ctx->scratch->ptr) + off;
@@ -1930,6 +1932,7 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
   if (oh < 0 || ow < 0) return fail(OHIP_E_SHAPE, "ohip_conv_transpose2d: pads exceed the un-cropped extent");
   if (d->n * d->cout * oh * ow > (int64_t)INT_MAX * 8 || d->h * d->w > INT_MAX / 2)
     return fail(OHIP_DECLINED, "ohip_conv_transpose2d: extent too large");
+  if (d->n * d->cout * oh * ow == 0) return OHIP_OK;
   std::lock_guard<std::mutex> lock(ctx->mu);
   ctx->counters.dispatches++;
   if (!w->phases.empty() && d->group == 1 && d->dil_h == 1 && d->dil_w == 1 && w->ph_sh == d->stride_h &&

@@ -1110,6 +1110,22 @@ def test_conv_transpose_joins_images(torch, ctx, xs, cout, launches, dt):
     assert _rel_err(y.float().cpu().numpy(), want) <= (F32_TOL if dt == "f32" else HALF_TOL)
 
 
+def test_conv_transpose_of_an_empty_batch(torch):
+    """No images: nothing to do, also on a context that never had scratch."""
+    from oxionnx_amd import _lib as L
+    from oxionnx_amd import device
+    ctx = device.HipContext(0)
+    geo = dict(strides=[2, 2], pads=[1, 1, 1, 1])
+    wt = ctx.weight_conv_transpose(np.ones((16, 8, 4, 4), np.float32), dtype=L.F32, **geo)
+    x = torch.ones((1, 16, 5, 5), device="cuda")
+    y = torch.full((1, 8, 10, 10), 7.0, device="cuda")
+    d = device._CONVT(0, 16, 5, 5, 8, 4, 4, 1, 2, 2, 1, 1, 1, 1, 1, 1, 0, 0, L.F32)
+    assert L.raw("ohip_conv_transpose2d")(ctx.h, d, x.data_ptr(), wt.handle, None, y.data_ptr()) == L.OK
+    ctx.sync()
+    assert bool((y == 7).all())
+    ctx.close()
+
+
 @pytest.mark.parametrize("a,b", [((2, 33, 2304), (2, 2304, 40)), ((3, 70, 1100), (3, 1100, 65)), ((5, 9, 4096), (1, 4096, 17))],
                          ids=str)
 @pytest.mark.parametrize("dt", ["f32", "f16"])
