@@ -87,6 +87,13 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
                    : kind == PlanKind::DenseF32 ? (int)(sizeof(kF32) / sizeof(TileCost))
                                                 : (int)(sizeof(kConv) / sizeof(TileCost));
   const int64_t nk = std::max<int64_t>(1, ((int64_t)kc + 7) / 8);
+  // How many of `s` slices have stages: the kernels give each ceil(nk / s), so
+  // the last of 6 slices of 10 stages would only write zeros for the reduction
+  // to read.  As many slices as that are as short.
+  auto filled = [&](int s) {
+    const uint32_t per = ((uint32_t)nk + s - 1) / s;
+    return (int)(((uint32_t)nk + per - 1) / per);
+  };
   if (plain_tile_id(override_tile)) return {1, override_tile};
   if (override_tile != 0 && override_tile != 10 && override_tile != 11) {   // a forced path that does not apply here
     override_tile = 0;
@@ -94,7 +101,7 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   }
   if (forced_splits()) return {may_split ? forced_splits() : 1, override_tile ? override_tile : may_split ? 10 : 9};
   if (override_tile != 0)
-    return {may_split ? (int)std::max<int64_t>(2, std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1)) : 1,
+    return {may_split ? std::max(2, filled((int)std::min<int64_t>(16, nk / 2 > 0 ? nk / 2 : 1))) : 1,
             may_split ? override_tile : override_tile == 11 ? 8 : 9};
   auto blocks = [&](int bp, int bq) {
     return (int64_t)(((uint32_t)P + (uint32_t)bp - 1) / (uint32_t)bp) * (((uint32_t)Q + (uint32_t)bq - 1) / (uint32_t)bq) *
@@ -117,9 +124,10 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     const float c = time(t, nb, nk);
     if (c < cost) { cost = c; best = {1, t.id}; }
     if (!may_split || (t.id != 9 && t.id != 8)) continue;
-    for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
-      const uint32_t per = ((uint32_t)nk + s - 1) / s;
+    for (const int most : {2, 3, 4, 6, 8, 12, 16}) {
+      const uint32_t per = ((uint32_t)nk + most - 1) / most;
       if (per < 2) break;
+      const int s = filled(most);
       const float cs = time(t, nb * s, per) + red.fix + red.per_slice * (float)s +
                        red.per_mb * (float)P * (float)Q * (float)batch * (float)s * 4e-6f;
       if (cs < cost) { cost = cs; best = {s, t.id == 9 ? 10 : 11}; }
