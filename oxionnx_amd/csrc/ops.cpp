@@ -176,8 +176,9 @@ static int activate(ohip_ctx* ctx) {
 // synchronises the stream first so no in-flight kernel still reads the old one.
 struct ScratchPlan {
   std::vector<size_t> sizes;
+  static size_t rounded(size_t b) { return (b + 255) & ~size_t(255); }
   size_t add(size_t b) {
-    sizes.push_back((b + 255) & ~size_t(255));
+    sizes.push_back(rounded(b));
     return sizes.size() - 1;
   }
   size_t total() const {
@@ -203,7 +204,9 @@ static int scratch_reserve(ohip_ctx* ctx, size_t bytes) {
 
 // Whether `bytes` of scratch cannot be had now because the context's stream is
 // capturing (growing waits for the stream and allocates): a call that can do
-// without, by running unsplit or in place, then does.
+// without, by running unsplit or in place, then does.  `bytes` are those that
+// the call reserves, rounded alike: the call that was run before its capture
+// left exactly that much.
 static bool scratch_frozen(ohip_ctx* ctx, size_t bytes) {
   if (bytes <= ctx->scratch_bytes) return false;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -1231,7 +1234,8 @@ extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, 
                       skinny_wins(d->dtype, M, N, b->kc, packed && !d->trans_a, sc.us);
   const bool gemv = M <= kMaxGemvM && !skinny;
   if (skinny) sc = TilePlan{1, 0};
-  if (sc.splits > 1 && scratch_frozen(ctx, split_ws_bytes((int)N, (int)M, sc.splits) + 256))
+  if (sc.splits > 1 && scratch_frozen(ctx, ScratchPlan::rounded(split_ws_bytes((int)N, (int)M, sc.splits)) +
+                                              (packed ? ScratchPlan::rounded((size_t)(M * kp) * eb) : 0)))
     sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, b->kc, ctx->tile_override, 1, false, false);
   const bool direct = !packed || (skinny && !d->trans_a);
 
@@ -1435,7 +1439,8 @@ static bool staged_f32_wins(ohip_ctx* ctx, const ohip_conv_desc* d, int64_t rows
   const bool k3 = d->kh == 3;
   const TilePlan sc = plan_tiles(PlanKind::DenseF32, (int)rows, (int)d->cout, (int)(d->kh * d->kw * (cp / 4)), 0);
   // its scratch has to fit an allocation-free call, and be there under capture
-  const size_t need = staged + split_ws_bytes((int)rows, (int)d->cout, sc.splits) + 512;
+  const size_t need =
+      ScratchPlan::rounded(staged) + ScratchPlan::rounded(split_ws_bytes((int)rows, (int)d->cout, sc.splits));
   if (noalloc ? need > kStaticScratchBytes : scratch_frozen(ctx, need)) return false;
   const float blocks = (float)(d->n * g.oh * ((g.ow + 63) / 64) * ((d->cout + 63) / 64)) * (g.ow <= 32 ? 0.55f : 1.0f);
   const float n = std::ceil(blocks / 256.0f), slabs = (float)((d->c + 7) / 8);
@@ -1604,8 +1609,7 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
                                        (int)G);
   // a static scratch too small for the slices' partial sums, or one that
   // cannot grow under capture: no split
-  const size_t sneed =
-      split_ws_bytes(sP, sQ, sc.splits) * (size_t)G + (stage ? (size_t)(d->n * sh_ * sw_ * cpt) * eb : 0) + 512;
+  const size_t sneed = plan.total() + ScratchPlan::rounded(split_ws_bytes(sP, sQ, sc.splits) * (size_t)G);
   if (!wk && !hsplits && sc.splits > 1 &&
       (noalloc ? sneed > kStaticScratchBytes : !norm && scratch_frozen(ctx, sneed)))
     sc = plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override, (int)G, false, false);
@@ -1884,7 +1888,7 @@ extern "C" int ohip_matmul(ohip_ctx* ctx, const ohip_matmul_desc* d, const void*
   const int forced = plain_tile_id(ctx->tile_override) ? ctx->tile_override : 0;
   TilePlan sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce), forced, (int)d->batch);
   if (sc.splits > 1 &&
-      scratch_frozen(ctx, plan.total() + split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch + 256))
+      scratch_frozen(ctx, plan.total() + ScratchPlan::rounded(split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch)))
     sc = plan_tiles(dense_kind(d->dtype), (int)N, (int)M, (int)(kp / ce), forced, (int)d->batch, false, false);
   size_t iw = sc.splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, sc.splits) * (size_t)d->batch) : SIZE_MAX;
   rc = scratch_reserve(ctx, plan.total());
@@ -2095,7 +2099,7 @@ extern "C" int ohip_qgemm(ohip_ctx* ctx, const ohip_qgemm_desc* d, const void* a
   size_t ir = d->n_azp > 1 ? plan.add((size_t)M * 4) : SIZE_MAX;
   const int ob = (d->out_kind == OHIP_QOUT_I32 || d->out_kind == OHIP_QOUT_F32) ? 4 : 1;
   TilePlan sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4);
-  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + split_ws_bytes((int)N, (int)M, sc.splits) + 256))
+  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + ScratchPlan::rounded(split_ws_bytes((int)N, (int)M, sc.splits))))
     sc = plan_tiles(PlanKind::Dense, (int)N, (int)M, b->kc, ctx->tile_override, 1, ob == 4, false);
   const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes((int)N, (int)M, splits)) : SIZE_MAX;
@@ -2226,7 +2230,7 @@ extern "C" int ohip_qconv2d(ohip_ctx* ctx, const ohip_qconv_desc* d, const void*
   size_t ix = stage ? plan.add((size_t)(d->n * d->h * d->w * cpt)) : SIZE_MAX;
   const int sP = nchw_out ? (int)rows : (int)coutg, sQ = nchw_out ? (int)coutg : (int)rows;
   TilePlan sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4);
-  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + split_ws_bytes(sP, sQ, sc.splits) + 256))
+  if (sc.splits > 1 && scratch_frozen(ctx, plan.total() + ScratchPlan::rounded(split_ws_bytes(sP, sQ, sc.splits))))
     sc = plan_tiles(PlanKind::Conv, sP, sQ, w->kc, ctx->tile_override, 1, ob == 4, false);
   const int splits = sc.splits;
   size_t iw = splits > 1 ? plan.add(split_ws_bytes(sP, sQ, splits)) : SIZE_MAX;

@@ -1222,6 +1222,48 @@ def test_capture_without_scratch(torch, op):
     ctx.close()
 
 
+@pytest.mark.parametrize("op", ["gemm", "matmul", "conv", "conv_transpose"])
+def test_capture_keeps_the_plan_of_the_call_before(torch, op):
+    """The call before its capture leaves exactly the scratch it needs: the
+    capture takes the same K slices and staging, so replays equal it bit for
+    bit."""
+    import ctypes
+
+    from oxionnx_amd import _lib as L
+    from oxionnx_amd.device import HipContext
+    ctx = HipContext(0)
+    rng = np.random.default_rng(8)
+    rand = lambda *shape: rng.uniform(-1, 1, shape).astype(np.float32)   # noqa: E731
+    if op == "gemm":
+        x, w = _dev(torch, rand(200, 8192)), ctx.weight_gemm(rand(8192, 301))
+        call = lambda: ctx.gemm(x, w)   # noqa: E731
+    elif op == "matmul":
+        x, z = _dev(torch, rand(3, 70, 4100)), _dev(torch, rand(3, 4100, 65))
+        call = lambda: ctx.matmul(x, z)   # noqa: E731
+    elif op == "conv":
+        x, w = _dev(torch, rand(4, 256, 14, 15)), ctx.weight_conv(rand(251, 256, 3, 3))
+        call = lambda: ctx.conv2d(x, w, pads=(1, 1, 1, 1))   # noqa: E731
+    else:
+        geo = dict(strides=(2, 2), pads=(1, 1, 1, 1))
+        x, w = _dev(torch, rand(1, 512, 16, 17)), ctx.weight_conv_transpose(rand(512, 255, 4, 4), **geo)
+        call = lambda: ctx.conv_transpose2d(x, w, **geo)   # noqa: E731
+    want = call()
+    torch.cuda.synchronize()
+    assert ctx.counters()["device_allocs"] > 0
+    g = ctypes.c_void_p()
+    L.check(L.lib().ohip_graph_begin(ctx.h))
+    y = call()
+    L.check(L.lib().ohip_graph_end(ctx.h, ctypes.byref(g)))
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        L.check(L.lib().ohip_graph_launch(g))
+        ctx.sync()
+        assert torch.equal(y, want)
+    L.lib().ohip_graph_destroy(g)
+    ctx.close()
+
+
 # one and two activation tiles, ragged weight tiles, partial last chunks, rows
 # of any alignment, with and without K slices (5000 x 40)
 @pytest.mark.parametrize("m", [2, 9, 16, 17, 32])
