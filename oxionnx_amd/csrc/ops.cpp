@@ -1965,23 +1965,34 @@ extern "C" int ohip_conv_transpose2d(ohip_ctx* ctx, const ohip_convt_desc* d, co
     const bool one = w->ph_all && oh % sh == 0 && ow % sw == 0 && prow > 0 && ph_one_launch() && !split_forced &&
                      d->n * prow <= INT_MAX / 2;
     const int64_t joined = one && prow >= 64 ? d->n : 1;
+    ScratchPlan plan;
+    size_t ix = plan.add((size_t)(d->n * d->h * d->w * cp) * eb);
+    bool may_split = true;
     auto plan_rows = [&](int64_t rows, const ohip_weight* ph, int phases) {
-      return plan_tiles(conv_kind(d->dtype), (int)rows, (int)d->cout, ph->kc, ctx->tile_override, phases);
+      return plan_tiles(conv_kind(d->dtype), (int)rows, (int)d->cout, ph->kc, ctx->tile_override, phases, false,
+                        may_split);
     };
     int max_splits = 1;
     TilePlan sc{1, 0};
-    if (one) {
-      sc = plan_rows(joined * prow, w->ph_all, (int)(sh * sw));
-      max_splits = sc.splits;
-    } else {
-      // (a phase's rows never exceed max_rows, but its plan may split more)
-      for (auto* ph : w->phases) max_splits = std::max(max_splits, plan_rows(max_rows, ph, 1).splits);
+    size_t slices = 0;   // bytes of partial sums
+    auto plan_all = [&] {
+      max_splits = 1;
+      if (one) {
+        sc = plan_rows(joined * prow, w->ph_all, (int)(sh * sw));
+        max_splits = sc.splits;
+        slices = split_ws_bytes((int)(joined * prow), (int)d->cout, max_splits) * (size_t)(sh * sw);
+      } else {
+        // (a phase's rows never exceed max_rows, but its plan may split more)
+        for (auto* ph : w->phases) max_splits = std::max(max_splits, plan_rows(max_rows, ph, 1).splits);
+        slices = split_ws_bytes((int)max_rows, (int)d->cout, max_splits);
+      }
+    };
+    plan_all();
+    if (max_splits > 1 && scratch_frozen(ctx, plan.total() + ScratchPlan::rounded(slices))) {
+      may_split = false;
+      plan_all();
     }
-    ScratchPlan plan;
-    size_t ix = plan.add((size_t)(d->n * d->h * d->w * cp) * eb);
-    size_t iw = max_splits > 1 ? plan.add(one ? split_ws_bytes((int)(joined * prow), (int)d->cout, max_splits) * (size_t)(sh * sw)
-                                              : split_ws_bytes((int)max_rows, (int)d->cout, max_splits))
-                               : SIZE_MAX;
+    size_t iw = max_splits > 1 ? plan.add(slices) : SIZE_MAX;
     rc = scratch_reserve(ctx, plan.total());
     if (rc) return rc;
     void* px = scratch_at(ctx, plan, ix);

@@ -1222,6 +1222,45 @@ def test_capture_without_scratch(torch, op):
     ctx.close()
 
 
+def test_capture_with_scratch_for_the_staging_alone(torch):
+    """A ConvTranspose captured on a context whose scratch holds its staged
+    input but not its K slices runs unsplit."""
+    import ctypes
+
+    from oxionnx_amd import _lib as L
+    from oxionnx_amd.device import HipContext
+    ctx = HipContext(0)
+    rng = np.random.default_rng(9)
+    ints = lambda *shape: rng.integers(-2, 3, shape).astype(np.float32)   # noqa: E731 (exact sums in any order)
+    warm_x, warm_w = _dev(torch, ints(1, 24, 20, 20)), ctx.weight_conv(ints(40, 24, 3, 3))
+    geo = dict(strides=(2, 2), pads=(1, 1, 1, 1))
+    x, w = _dev(torch, ints(1, 512, 16, 16)), ctx.weight_conv_transpose(ints(512, 200, 4, 4), **geo)
+    ctx.conv2d(warm_x, warm_w, strides=(2, 2))   # 1 MiB, the least a context takes: the input above is half of it
+    y = torch.zeros((1, 200, 32, 32), device="cuda")
+    torch.cuda.synchronize()
+    allocs = ctx.counters()["device_allocs"]
+    assert allocs > 0
+    g = ctypes.c_void_p()
+    L.check(L.lib().ohip_graph_begin(ctx.h))
+    ctx.conv_transpose2d(x, w, out=y, **geo)
+    L.check(L.lib().ohip_graph_end(ctx.h, ctypes.byref(g)))
+    assert ctx.counters()["device_allocs"] == allocs
+    got = []
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        L.check(L.lib().ohip_graph_launch(g))
+        ctx.sync()
+        got.append(y.clone())
+    y.zero_()
+    ctx.conv_transpose2d(x, w, out=y, **geo)   # eager: with K slices, in a larger scratch
+    ctx.sync()
+    assert ctx.counters()["device_allocs"] > allocs
+    assert bool(y.any()) and all(torch.equal(v, y) for v in got)
+    L.lib().ohip_graph_destroy(g)
+    ctx.close()
+
+
 @pytest.mark.parametrize("op", ["gemm", "matmul", "conv", "conv_transpose"])
 def test_capture_keeps_the_plan_of_the_call_before(torch, op):
     """The call before its capture leaves exactly the scratch it needs: the
