@@ -1611,7 +1611,7 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   // cannot grow under capture: no split
   const size_t sneed = plan.total() + ScratchPlan::rounded(split_ws_bytes(sP, sQ, sc.splits) * (size_t)G);
   if (!wk && !hsplits && sc.splits > 1 &&
-      (noalloc ? sneed > kStaticScratchBytes : !norm && scratch_frozen(ctx, sneed)))
+      (noalloc ? sneed > kStaticScratchBytes : scratch_frozen(ctx, sneed)))
     sc = plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override, (int)G, false, false);
   const int splits = sc.splits;
   if (norm && splits == 1 && !wk) {   // counted again by the two-step path's plain call
