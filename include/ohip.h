@@ -229,12 +229,14 @@ int ohip_conv2d(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohi
                 const void* bias, void* y);
 /* ohip_conv2d without device allocation.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * kernels and results as ohip_conv2d; the NCHW staging copy and the split-K
- * partial sums live in a static 32 MiB device array per GPU instead of the
- * context's growable scratch.  A call that fits there only unsplit, or only
- * unstaged, runs so; one needing more scratch still returns OHIP_E_NOMEM and
- * launches nothing.  Every call on one GPU shares the array,
+ * capture, tight serving loops, harnesses that forbid hipMalloc).  The
+ * kernels of ohip_conv2d; the NCHW staging copy and the split-K partial sums
+ * live in a static 32 MiB device array per GPU instead of the context's
+ * growable scratch.  Where they fit the results are ohip_conv2d's, bit for
+ * bit.  K slices that do not fit are left out, and an f32 NCHW 3x3 / 1x1
+ * stride-1 convolution whose staging does not fit reads its input in place
+ * (the same products, summed in another order); any other call needing more
+ * scratch returns OHIP_E_NOMEM and launches nothing.  Every call on one GPU shares the array,
  * so calls that overlap on one GPU (other streams or contexts) race. */
 int ohip_conv2d_noalloc(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohip_weight* w,
                         const void* bias, void* y);

@@ -1556,10 +1556,14 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   const int64_t staged_w = fused_pad ? d->w + d->pad_l + d->pad_r : d->w;
   const int64_t staged_bytes =
       (fused_pad ? (d->h + d->pad_t + d->pad_b) * (d->w + d->pad_l + d->pad_r) : d->h * d->w) * cpt * eb;
+  // So does a call whose staged copy cannot be had.
+  auto fits = [&](size_t bytes) { return noalloc ? bytes <= kStaticScratchBytes : !scratch_frozen(ctx, bytes); };
   if (!norm && !direct && !fewout && d->dtype == OHIP_F32 && G == 1 && d->in_layout == OHIP_NCHW &&
-      nchw_f32_allowed() && conv_nchw_f32_supported(a) && !wk_plan(ctx, d, G, staged_w, g, staged_bytes) &&
-      halo_plan(ctx, d, G, staged_w, g, (int)(cp / ce), staged_bytes) == 0 &&
-      !staged_f32_wins(ctx, d, rows, g, cp, (size_t)(d->n * staged_bytes), noalloc)) {
+      nchw_f32_allowed() && conv_nchw_f32_supported(a) &&
+      (!fits(ScratchPlan::rounded((size_t)(d->n * staged_bytes))) ||
+       (!wk_plan(ctx, d, G, staged_w, g, staged_bytes) &&
+        halo_plan(ctx, d, G, staged_w, g, (int)(cp / ce), staged_bytes) == 0 &&
+        !staged_f32_wins(ctx, d, rows, g, cp, (size_t)(d->n * staged_bytes), noalloc)))) {
     ctx->counters.contraction_launches++;
     hipError_t e = run_conv_nchw_f32(static_cast<const float*>(x), static_cast<const float*>(w->data),
                                      static_cast<const float*>(bias), static_cast<float*>(y), a, ctx->stream);
@@ -1599,19 +1603,19 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
   // the halo-patch kernel (the input patch staged once per channel slab for
   // all nine taps) instead of the engine's im2col gather.
   const bool wk = wk_plan(ctx, d, G, sw_, g, (int64_t)(sh_ * sw_ * cpt * eb));
-  const int hsplits = wk ? 0 : halo_plan(ctx, d, G, sw_, g, (int)(cp / ce), (int64_t)(sh_ * sw_ * cpt * eb));
+  int hsplits = wk ? 0 : halo_plan(ctx, d, G, sw_, g, (int)(cp / ce), (int64_t)(sh_ * sw_ * cpt * eb));
   if (nhwc_pad && !hsplits && !wk)
     return fail(OHIP_DECLINED, "ohip_conv2d: a reflect / edge Pad on an NHWC input needs the halo-patch path");
+  // a static scratch too small for the slices' partial sums, or one that
+  // cannot grow under capture: no split
+  auto slices_fit = [&](int s) { return fits(plan.total() + ScratchPlan::rounded(split_ws_bytes(sP, sQ, s) * (size_t)G)); };
+  if (hsplits > 1 && !slices_fit(hsplits)) hsplits = 1;
   // groups share one launch (the group on the grid z)
   TilePlan sc = wk        ? TilePlan{1, 0}
                 : hsplits ? TilePlan{hsplits, 0}
                           : plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override,
                                        (int)G);
-  // a static scratch too small for the slices' partial sums, or one that
-  // cannot grow under capture: no split
-  const size_t sneed = plan.total() + ScratchPlan::rounded(split_ws_bytes(sP, sQ, sc.splits) * (size_t)G);
-  if (!wk && !hsplits && sc.splits > 1 &&
-      (noalloc ? sneed > kStaticScratchBytes : scratch_frozen(ctx, sneed)))
+  if (!wk && !hsplits && sc.splits > 1 && !slices_fit(sc.splits))
     sc = plan_tiles(conv_kind(d->dtype), sP, sQ, (int)(d->kh * d->kw * (cp / ce)), ctx->tile_override, (int)G, false, false);
   const int splits = sc.splits;
   if (norm && splits == 1 && !wk) {   // counted again by the two-step path's plain call
@@ -1633,6 +1637,10 @@ static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, co
                        : SIZE_MAX;
   const size_t ity = wk_mom ? plan.add((size_t)(d->n * d->cout * ohw) * eb) : SIZE_MAX;
   const size_t imom = wk_mom ? plan.add((size_t)(d->n * d->cout * (ohw / 64)) * 2 * 4) : SIZE_MAX;
+  if (wk && norm && !fits(plan.total())) {   // no room for what the fused norm reads: two steps
+    ctx->counters.dispatches--;
+    return kNormTwoStep;
+  }
   char* sbase = nullptr;
   rc = call_scratch(ctx, plan.total(), noalloc, &sbase);
   if (rc) return rc;

@@ -1175,7 +1175,7 @@ def test_captured_scratch_outlives_growth(torch):
     ctx.close()
 
 
-@pytest.mark.parametrize("op", ["gemm", "conv", "qgemm"])
+@pytest.mark.parametrize("op", ["gemm", "conv", "halo_conv", "qgemm"])
 def test_capture_without_scratch(torch, op):
     """A call that needs scratch only for its K slices or its staging is
     captured on a context that has none: unsplit, or in place."""
@@ -1189,6 +1189,11 @@ def test_capture_without_scratch(torch, op):
         x = _dev(torch, rng.integers(-3, 4, (4, 128, 14, 14)).astype(np.float32))
         w = ctx.weight_conv(rng.integers(-3, 4, (64, 128, 3, 3)).astype(np.float32), dtype=L.F32)
         y = torch.empty((4, 64, 14, 14), dtype=torch.float32, device="cuda")
+        call = lambda: ctx.conv2d(x, w, pads=(1, 1, 1, 1), out=y)
+    elif op == "halo_conv":
+        x = _dev(torch, rng.integers(-3, 4, (1, 192, 128, 128)).astype(np.float32))
+        w = ctx.weight_conv(rng.integers(-3, 4, (192, 192, 3, 3)).astype(np.float32), dtype=L.F32)
+        y = torch.empty((1, 192, 128, 128), dtype=torch.float32, device="cuda")
         call = lambda: ctx.conv2d(x, w, pads=(1, 1, 1, 1), out=y)
     elif op == "gemm":
         x = _dev(torch, rng.integers(-3, 4, (64, 4096)).astype(np.float32)).half()

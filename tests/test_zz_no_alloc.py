@@ -77,3 +77,20 @@ def test_noalloc_rejects_more_scratch_than_the_static_array(torch, ctx):
     with pytest.raises(L.OhipError) as e:
         ctx.conv2d(x, wt, None, out=out, noalloc=True)
     assert e.value.code == L.E_NOMEM and "static" in str(e.value)
+
+
+# a halo-path f32 convolution whose K slices, or whose staged input, exceed
+# 32 MiB: unsplit, or in place (whole numbers: the same sums in any order)
+@pytest.mark.parametrize("xs,cout", [((1, 192, 128, 128), 192), ((9, 64, 128, 128), 64)], ids=["slices", "staging"])
+def test_noalloc_halo_without_room(torch, ctx, xs, cout):
+    rng = np.random.default_rng(xs[1])
+    x = torch.from_numpy(rng.integers(-3, 4, xs).astype(np.float32)).cuda()
+    wt = ctx.weight_conv(rng.integers(-3, 4, (cout, xs[1], 3, 3)).astype(np.float32))
+    want = ctx.conv2d(x, wt, pads=(1, 1, 1, 1))
+    got = torch.full_like(want, float("nan"))
+    torch.cuda.synchronize()
+    ctx.reset_counters()
+    ctx.conv2d(x, wt, pads=(1, 1, 1, 1), out=got, noalloc=True)
+    torch.cuda.synchronize()
+    assert ctx.counters()["device_allocs"] == 0
+    assert torch.equal(got, want)
