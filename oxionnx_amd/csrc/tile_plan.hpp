@@ -24,7 +24,7 @@ inline int forced_splits() {
 }
 
 // A block tile and the K slices it runs with (splits > 1: tile 10 or 11);
-// us: its estimated time without the launch (0: not estimated).
+// us: its estimated time without the launch (0: a forced plan, not estimated).
 struct TilePlan {
   int splits, tile;
   float us = 0.0f;
@@ -107,13 +107,14 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     return (int64_t)(((uint32_t)P + (uint32_t)bp - 1) / (uint32_t)bp) * (((uint32_t)Q + (uint32_t)bq - 1) / (uint32_t)bq) *
            batch;
   };
-  if (nk > 16 && blocks(256, 256) >= 256) return {1, 16};
   auto time = [&](const TileCost& t, int64_t nb, int64_t stages) {
     const uint32_t ncu = (uint32_t)std::min<int64_t>((nb + 255) >> 8, 1 << 24), res = (uint32_t)t.res;
     const uint32_t q = ncu / res, rem = ncu - q * res;
     return t.fix * (float)(q + (rem ? 1 : 0)) +
            (float)stages * ((float)q * std::max(t.lat, (float)t.res * t.bw) + (rem ? std::max(t.lat, (float)rem * t.bw) : 0.0f));
   };
+  if (nk > 16 && blocks(256, 256) >= 256)   // (the convolutions' table has no tile 16: the dense cost)
+    return {1, 16, time(kind == PlanKind::DenseF32 ? kF32[6] : kDense[7], blocks(256, 256), nk)};
   TilePlan best{1, 1};
   float cost = INFINITY;
   for (int i = 0; i < ntab; ++i) {

@@ -1175,6 +1175,24 @@ def test_captured_scratch_outlives_growth(torch):
     ctx.close()
 
 
+def test_large_f32_convolution_reads_its_input_in_place(torch):
+    """1x64x256x256 -> 64, 3x3: 64 us in place, 180 staged on the engine's
+    largest tile (64 of its 256 columns full); no scratch is taken."""
+    from oxionnx_amd.device import HipContext
+    ctx = HipContext(0)
+    rng = np.random.default_rng(6)
+    x = _dev(torch, rng.uniform(-1, 1, (1, 64, 256, 256)).astype(np.float32))
+    w = rng.normal(0, 0.05, (64, 64, 3, 3)).astype(np.float32)
+    wt = ctx.weight_conv(w)
+    torch.cuda.synchronize()
+    allocs = ctx.counters()["device_allocs"]
+    y = ctx.conv2d(x, wt, pads=(1, 1, 1, 1))
+    assert ctx.counters()["device_allocs"] == allocs
+    want = torch.nn.functional.conv2d(x.cpu().double(), torch.from_numpy(w).double(), padding=1).numpy()
+    assert _rel_err(y.cpu().numpy(), want) <= F32_TOL
+    ctx.close()
+
+
 @pytest.mark.parametrize("op", ["gemm", "conv", "halo_conv", "qgemm"])
 def test_capture_without_scratch(torch, op):
     """A call that needs scratch only for its K slices or its staging is
