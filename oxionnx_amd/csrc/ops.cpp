@@ -1183,26 +1183,6 @@ static bool rows_direct(const void* a, int64_t k, int64_t ld, int eb, int trans)
 }
 
 // ------------------------------------------------------------------ float GEMM
-static const int kMaxGemvM = 8;
-static const int kMaxSkinnyM = 32;
-// Whether a few rows run the skinny kernel instead of GEMV (up to
-// kMaxGemvM) or the engine (estimated at tile_us): estimated times in us past
-// the launch, fitted to 16 weights of 77-11008 rows and 333-25088 columns at
-// 1-32 rows, f16 and f32 (graph replay).  The skinny kernel's waves walk K in
-// steps of 256 chunks a block, at the memory's rate if that is slower; GEMV
-// reads the activations again for every weight row or two.  Rows that GEMV or
-// the engine would pack first cost them a launch (2.5).  5x768x3072 f16 6.6 ->
-// 4.2 us, 8x4096x4096 38 -> 9.4, 12x512x1024 f32 11 -> 5.0, 2x777x1001 f16
-// 6.2 -> 4.1; 5x25088x512 stays GEMV (11.3 against 34: 32 blocks).
-static bool skinny_wins(int dtype, int64_t m, int64_t n, int64_t kc, bool pack, float tile_us) {
-  const bool f32 = dtype == OHIP_F32;
-  const float steps = (float)((kc + 31) / 32), mb = (float)n * (float)kc * 16e-6f, rows = (float)m;
-  const float step = f32 ? .29f + .0125f * rows : .25f + .0115f * rows;
-  const float rate = f32 ? 5.4f : steps >= 16.0f ? 6.5f : 4.5f;   // MB a us
-  const float skinny = std::max(step * steps, mb / rate);
-  const float other = m <= kMaxGemvM ? mb / 7.0f + rows * (.33f + (f32 ? .02f : .04f) * mb) : tile_us + .2f;
-  return skinny < other + (pack ? 2.5f : 0.0f);
-}
 static PlanKind dense_kind(int dtype) { return dtype == OHIP_F32 ? PlanKind::DenseF32 : PlanKind::Dense; }
 static PlanKind conv_kind(int dtype) { return dtype == OHIP_F32 ? PlanKind::DenseF32 : PlanKind::Conv; }
 
@@ -1231,7 +1211,7 @@ extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, 
   TilePlan sc = M <= kMaxGemvM ? TilePlan{1, ctx->tile_override}
                                : plan_tiles(dense_kind(d->dtype), (int)N, (int)M, b->kc, ctx->tile_override);
   const bool skinny = M <= kMaxSkinnyM && ctx->tile_override == 0 && !forced_splits() &&
-                      skinny_wins(d->dtype, M, N, b->kc, packed && !d->trans_a, sc.us);
+                      skinny_wins(d->dtype == OHIP_F32, M, N, b->kc, packed && !d->trans_a, sc);
   const bool gemv = M <= kMaxGemvM && !skinny;
   if (skinny) sc = TilePlan{1, 0};
   if (sc.splits > 1 && scratch_frozen(ctx, ScratchPlan::rounded(split_ws_bytes((int)N, (int)M, sc.splits)) +

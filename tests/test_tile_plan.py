@@ -16,11 +16,15 @@ extern "C" float plan(int kind, int P, int Q, int kc, int forced, int batch, int
   out[1] = t.tile;
   return t.us;
 }
+extern "C" int skinny(int f32, int m, int n, int kc, int pack) {
+  const TilePlan t = m <= kMaxGemvM ? TilePlan{1, 0} : plan_tiles(f32 ? PlanKind::DenseF32 : PlanKind::Dense, n, m, kc, 0);
+  return skinny_wins(f32 != 0, m, n, kc, pack != 0, t);
+}
 """
 
 
 @pytest.fixture(scope="module")
-def plan(tmp_path_factory):
+def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("plan")
     (d / "p.cpp").write_text(SOURCE)
     so = str(d / "p.so")
@@ -28,7 +32,11 @@ def plan(tmp_path_factory):
                     str(d / "p.cpp"), "-o", so], check=True)
     lib = ctypes.CDLL(so)
     lib.plan.restype = ctypes.c_float
+    return lib
 
+
+@pytest.fixture(scope="module")
+def plan(lib):
     def call(kind, p, q, kc, forced=0, batch=1, wide=0):
         out = (ctypes.c_int * 2)()
         us = lib.plan(kind, p, q, kc, forced, batch, wide, out)
@@ -63,3 +71,21 @@ def test_every_plan_has_an_estimate(plan, kind, k, rate):
         tiles.add(tile)
         assert us >= 2.0 * p * q * kc * k / rate, (p, q, kc, tile, us)
     assert 16 in tiles
+
+
+# (type, rows, K, N): skinny kernel against GEMV / engine in us, both timed
+FEW_ROWS = [("f16", 2, 768, 3072, 4.8, 5.2), ("f16", 2, 1024, 8192, 6.0, 7.2), ("f16", 16, 2048, 70001, 78.7, 85.5),
+            ("f16", 8, 4096, 4096, 9.6, 30.2), ("f16", 9, 4096, 4096, 9.5, 11.7),
+            ("f16", 32, 768, 768, 5.6, 8.1), ("f16", 24, 2048, 8192, 13.3, 11.7), ("f16", 32, 2048, 8192, 14.6, 12.4),
+            ("f16", 24, 4096, 11008, 31.8, 22.3), ("f16", 32, 4096, 11008, 35.7, 22.7), ("f16", 24, 4096, 4096, 13.2, 12.3),
+            ("f16", 32, 3072, 768, 11.4, 8.9), ("f16", 32, 2048, 70001, 114.8, 87.4), ("f16", 2, 2048, 70001, 55.7, 49.1),
+            ("f32", 9, 4096, 11008, 44.8, 64.6), ("f32", 32, 1024, 8192, 16.7, 17.7), ("f32", 16, 4096, 4096, 20.7, 26.4), ("f32", 32, 768, 3072, 8.6, 11.2),
+            ("f32", 24, 4096, 11008, 73.0, 65.9), ("f32", 32, 4096, 32000, 231.9, 152.0), ("f32", 32, 2048, 2048, 16.4, 13.3),
+            ("f32", 2, 768, 30522, 25.7, 19.1), ("f32", 2, 1024, 50257, 45.3, 35.7), ("f32", 16, 2048, 70001, 172.0, 916.3)]
+
+
+@pytest.mark.parametrize("case", FEW_ROWS, ids=lambda c: "%s-%dx%dx%d" % c[:4])
+def test_few_rows_take_the_faster_kernel(lib, case):
+    dt, m, k, n, skinny, other = case
+    per = 4 if dt == "f32" else 8
+    assert bool(lib.skinny(int(dt == "f32"), m, n, -(-k // per), int(k % per != 0))) == (skinny < other)
