@@ -1,4 +1,4 @@
-// MFMA contraction kernels, bf16, implicit im2col.
+// MFMA contraction kernels, bf16, implicit im2col, pixels on X (NCHW outputs).
 #define OHIP_OP Op::BF16
 #define OHIP_OUT __bf16
 #define OHIP_SUFFIX bf16

@@ -1,4 +1,4 @@
-// MFMA contraction kernels, f16, implicit im2col.
+// MFMA contraction kernels, f16, implicit im2col, pixels on X (NCHW outputs).
 #define OHIP_OP Op::F16
 #define OHIP_OUT _Float16
 #define OHIP_SUFFIX f16

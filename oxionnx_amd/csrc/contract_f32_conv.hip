@@ -1,4 +1,4 @@
-// MFMA contraction kernels, f32, implicit im2col.
+// MFMA contraction kernels, f32, implicit im2col, pixels on X (NCHW outputs).
 #define OHIP_OP Op::F32
 #define OHIP_OUT float
 #define OHIP_SUFFIX f32

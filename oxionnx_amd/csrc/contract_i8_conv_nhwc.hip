@@ -1,0 +1,7 @@
+// MFMA contraction kernels, i8, implicit im2col, pixels on Y (NHWC outputs).
+#define OHIP_OP Op::I8
+#define OHIP_OUT void
+#define OHIP_SUFFIX i8
+#define OHIP_PART 3
+#define OHIP_QUANT 1
+#include "contract.inc"

@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(Wt::kThreads) wk_conv_kernel(const HaloGeo g, 
   if (wave >= Wt::NPT) return;
   // wave pt adds the partial tiles of k-steps 0 .. KSN - 1 in that order and
   // finishes its 32 pixels x 32 channels
-  const OutAddr out = epi.addr();
+  const auto out = epi.addr();
   const int pixl = pix0 + pt * 32;
   const int jl = Wt::PIX_ON_X ? co0 + (lane & 31) : pixl + (lane & 31);
   typename Epi::PreJ pj;

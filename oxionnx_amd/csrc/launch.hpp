@@ -82,7 +82,7 @@ template <class T> __device__ __forceinline__ uint32_t out_bits(T v) {
 // Float output: v = acc * alpha; v = v + beta * bias; act; round to OutT.
 // alpha == 1 multiplies exactly, and a missing bias adds -0.0, the exact
 // additive identity, so neither needs a branch.
-template <class OutT> struct FloatEpi {
+template <class OutT, bool GENERAL = true> struct FloatEpi {
   OutAddr out;
   float alpha, beta;
   const OutT* bias;
@@ -92,6 +92,10 @@ template <class OutT> struct FloatEpi {
   int act;
   float lo, hi;
 
+  static constexpr bool kGeneral = GENERAL;
+  using Addr = std::conditional_t<GENERAL, OutAddr, PlainAddr>;
+  using Plain = FloatEpi<OutT, false>;   // the same fields
+  Plain plain() const { return __builtin_bit_cast(Plain, *this); }
   static constexpr int kStageBytes = sizeof(OutT) <= 2 ? (int)sizeof(OutT) : 0;
   static constexpr bool kStageWide = sizeof(OutT) == 4;   // f32 outputs stage as 4-byte elements
   // finish() reduces to acc + the row term: alpha is 1 (an exact multiply),
@@ -105,13 +109,13 @@ template <class OutT> struct FloatEpi {
            act == ACT_NONE;
   }
   __device__ __forceinline__ int out_bytes() const { return (int)sizeof(OutT); }
-  __device__ __forceinline__ OutAddr addr() const { return out; }
+  __device__ __forceinline__ Addr addr() const { return Addr{out}; }
   // 16-byte chunks of output rows: no chunk straddles two images
-  __device__ __forceinline__ bool staged_ok() const {
+  __host__ __device__ __forceinline__ bool staged_ok() const {
     return out.stage && out.vec && ((uintptr_t)out.y % 16 == 0) && ((out.sj * (int64_t)sizeof(OutT)) % 16 == 0) &&
            (out.bstride == 0 || (out.ohw * (int)sizeof(OutT) % 16 == 0 && out.bstride * (int64_t)sizeof(OutT) % 16 == 0));
   }
-  __device__ __forceinline__ bool staged_wide_ok() const { return sizeof(OutT) == 4 && staged_ok(); }
+  __host__ __device__ __forceinline__ bool staged_wide_ok() const { return sizeof(OutT) == 4 && staged_ok(); }
 
   struct PreI { float b[4]; };    // beta * bias per row (BIAS_I, BIAS_SCALAR), else -0
   struct PreJ { float b; };       // beta * bias per column (BIAS_J), else -0
@@ -197,7 +201,7 @@ template <class OutT> struct FloatEpi {
 // true value fits int32 (the host gate guarantees it).  Requantisation then
 // follows SatRange::requantize: f64 product with the f32 combined scale, + zp,
 // round half to even, clamp.
-struct QuantEpi {
+template <bool GENERAL = true> struct QuantEpi {
   OutAddr out;
   int w_on_i;               // weight channel index is i (else j)
   const int32_t* colsum;    // per weight channel
@@ -216,6 +220,10 @@ struct QuantEpi {
   // on i, a per-tensor correction factor, a u8 / i8 output, with or without the byte table), whose
   // finish needs only the row terms; the staged epilogue then runs
   // finish_simple, the same arithmetic with no uniform branches
+  static constexpr bool kGeneral = GENERAL;
+  using Addr = std::conditional_t<GENERAL, OutAddr, PlainAddr>;
+  using Plain = QuantEpi<false>;
+  Plain plain() const { return __builtin_bit_cast(Plain, *this); }
   static constexpr bool kHasSimple = true;
   // Mode 2 (4-byte outputs): the raw int32 form (MatMulInteger) likewise.
   // Returns 1 for the plain form, 2 for a u8 / i8 form with the byte table
@@ -230,12 +238,12 @@ struct QuantEpi {
   static constexpr int kStageBytes = 1;
   static constexpr bool kStageWide = true;   // int32 / f32 outputs stage as 4-byte elements
   __device__ __forceinline__ int out_bytes() const { return (out_kind == QOUT_U8 || out_kind == QOUT_I8) ? 1 : 4; }
-  __device__ __forceinline__ OutAddr addr() const { return out; }
-  __device__ __forceinline__ bool staged_ok() const {
+  __device__ __forceinline__ Addr addr() const { return Addr{out}; }
+  __host__ __device__ __forceinline__ bool staged_ok() const {
     return out.stage && (out_kind == QOUT_U8 || out_kind == QOUT_I8) && out.vec && ((uintptr_t)out.y % 16 == 0) &&
            (out.sj % 16 == 0) && (out.bstride == 0 || (out.ohw % 16 == 0 && out.bstride % 16 == 0));
   }
-  __device__ __forceinline__ bool staged_wide_ok() const {
+  __host__ __device__ __forceinline__ bool staged_wide_ok() const {
     return out.stage && (out_kind == QOUT_I32 || out_kind == QOUT_F32) && out.vec && ((uintptr_t)out.y % 16 == 0) &&
            (out.sj % 4 == 0) && (out.bstride == 0 || (out.ohw % 4 == 0 && out.bstride % 4 == 0));
   }
@@ -437,9 +445,16 @@ inline hipError_t launch_reduce(const void* ws, int splits, int P, int Q, const 
   const int64_t groups = (int64_t)(Pp / 4) * Q;
   if (groups > 0x7fffffff) return hipErrorInvalidValue;   // the reduction indexes groups in 32 bits
   const unsigned grid = (unsigned)std::min<int64_t>((groups + 255) / 256, 65535 * 4);
-  const int batch = epi.out.batch > 1 ? epi.out.batch : 1;
-  hipLaunchKernelGGL((split_reduce_kernel<T, V, Epi>), dim3(grid, 1, (unsigned)batch), dim3(256), 0, st,
-                     reinterpret_cast<const T*>(ws), splits, P, Pp, Q, epi);
+  auto go = [&](const auto& e, int batch) {
+    hipLaunchKernelGGL((split_reduce_kernel<T, V, std::decay_t<decltype(e)>>), dim3(grid, 1, (unsigned)batch), dim3(256),
+                       0, st, reinterpret_cast<const T*>(ws), splits, P, Pp, Q, e);
+  };
+  if (epi.out.batch > 1 || epi.out.rw > 0) {
+    if constexpr (Epi::kGeneral) go(epi, epi.out.batch > 1 ? epi.out.batch : 1);
+    else return hipErrorInvalidValue;
+  } else {
+    go(epi.plain(), 1);
+  }
   return hipGetLastError();
 }
 
@@ -539,18 +554,20 @@ inline hipError_t launch_wk(const HaloGeo& g, const Epi& epi, int P, int Q, void
 // XX / XY: the X / Y operand holds u8 activations that the MFMA reads as
 // int8 after XOR 0x80.
 template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
-inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
-                             int splits, void* split_ws, hipStream_t st) {
-  if (splits > 1) {
-    // OHIP_SPLIT_TILE=12/13/14 runs the slices on that deeper-pipelined tile (a measurement switch)
-    static const int sv = [] { const char* e = std::getenv("OHIP_SPLIT_TILE"); return e ? std::atoi(e) : 0; }();
-    if (sv == 12) return launch_split_on<O, XX, XY, T128d4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-    if (sv == 13) return launch_split_on<O, XX, XY, T64d8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-    if (sv == 14) return launch_split_on<O, XX, XY, T128x4w4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-    if (tile == 11)
-      return launch_split_on<O, XX, XY, T128w8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-    return launch_split_on<O, XX, XY, T64s4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
-  }
+inline hipError_t launch_split(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
+                               int splits, void* split_ws, hipStream_t st) {
+  // OHIP_SPLIT_TILE=12/13/14 runs the slices on that deeper-pipelined tile (a measurement switch)
+  static const int sv = [] { const char* e = std::getenv("OHIP_SPLIT_TILE"); return e ? std::atoi(e) : 0; }();
+  if (sv == 12) return launch_split_on<O, XX, XY, T128d4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
+  if (sv == 13) return launch_split_on<O, XX, XY, T64d8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
+  if (sv == 14) return launch_split_on<O, XX, XY, T128x4w4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
+  if (tile == 11)
+    return launch_split_on<O, XX, XY, T128w8>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
+  return launch_split_on<O, XX, XY, T64s4>(lx, ly, epi, P, Q, kc, splits, split_ws, st);
+}
+template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
+inline hipError_t launch_unsplit(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
+                                 hipStream_t st) {
   switch (tile) {   // the caller's plan (plan_tiles)
     case 2: return launch_tile<O, XX, XY, T128>(lx, ly, epi, P, Q, kc, st);
     case 3: return launch_tile<O, XX, XY, T256x128>(lx, ly, epi, P, Q, kc, st);
@@ -567,6 +584,12 @@ inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, 
     case 18: return launch_tile<O, XX, XY, T192x256>(lx, ly, epi, P, Q, kc, st);
     default: return launch_tile<O, XX, XY, T64>(lx, ly, epi, P, Q, kc, st);
   }
+}
+template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
+inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
+                             int splits, void* split_ws, hipStream_t st) {
+  if (splits > 1) return launch_split<O, XX, XY>(lx, ly, epi, P, Q, kc, tile, splits, split_ws, st);
+  return launch_unsplit<O, XX, XY>(lx, ly, epi, P, Q, kc, tile, st);
 }
 
 // Per-slice pads (Im2colNHWC::zpt / zpl) hold four entries, indexed by the
@@ -614,8 +637,8 @@ inline FloatEpi<OutT> make_float_epi(const FloatOut& o) {
   return e;
 }
 
-inline QuantEpi make_quant_epi(const QuantOut& o) {
-  QuantEpi e;
+inline QuantEpi<> make_quant_epi(const QuantOut& o) {
+  QuantEpi<> e;
   e.out = make_out_addr(o);
   e.w_on_i = o.w_on_i; e.colsum = o.colsum; e.flip = o.flip; e.bias = o.bias; e.ca = o.ca;
   e.ca_rows = o.ca_rows; e.comb = o.comb; e.n_comb = o.n_comb; e.out_kind = o.out_kind;

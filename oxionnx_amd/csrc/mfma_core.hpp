@@ -418,6 +418,20 @@ struct OutAddr {
     return zsw > 0 ? (int64_t)(z / zsw) * zrow + (int64_t)(z % zsw) * zstride : (int64_t)z * zstride;
   }
 };
+// The map of one contraction without batch slices and strided rows.  The
+// epilogues come in both forms (kGeneral; the host chooses, contract.inc): the
+// plain one also leaves out the ragged flush.  A kernel that writes whole
+// aligned rows pays for both even where it never takes them: f16 256x768x3072
+// 0.3 of 7.8 us, 384x768x768 0.3 of 7.5 (graph replay), the f16 generator's
+// forward about 1 %.
+struct PlainAddr : OutAddr {
+  __device__ __forceinline__ int64_t row(int i) const {
+    if (bstride == 0) return (int64_t)i * si;
+    const int n = (int)(((uint64_t)(uint32_t)i * ohw_mul) >> ohw_shift);
+    return (int64_t)n * bstride + (int64_t)(i - n * ohw) * si;
+  }
+  __device__ __forceinline__ int64_t slice_offset() const { return 0; }
+};
 
 // Division by an invariant d >= 1 for dividends below 2^31: with
 // s = ceil(log2 d) and m = ceil(2^(31+s) / d) (which fits 32 bits),
@@ -433,7 +447,8 @@ inline void magic_div(int d, uint32_t* mul, int* shift) {
 
 // Stores the four outputs (rows i .. i+3, column j) whose bit patterns are
 // bits[r]; row = out.row(i).
-__device__ __forceinline__ void store_group(const OutAddr& out, int eb, int64_t row, int i, int j,
+template <class Addr>
+__device__ __forceinline__ void store_group(const Addr& out, int eb, int64_t row, int i, int j,
                                             const uint32_t (&v)[4]) {
   if (j >= out.Q) return;
   const int64_t cj = (int64_t)j * out.sj;
@@ -481,7 +496,7 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   using A4 = typename OpT<O>::Out4;
   const int ibase = p0 + wp * Tl::TP * 32 + (lane >> 5) * 4;
   const int jbase = q0 + wq * Tl::TQ * 32 + (lane & 31);
-  OutAddr out = epi.addr();
+  auto out = epi.addr();
   out.y += out.slice_offset();
 
   // the per-column epilogue terms, loaded once for all of this lane's rows
@@ -497,7 +512,8 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   // Mode 1 stages the epilogue's narrow output (1 or 2 bytes); mode 2 stages
   // 4-byte outputs (int32, f32) when the tile's stage buffers hold them.
   // `ragged`: the output rows are not runs of aligned 16-byte chunks (an odd
-  // N or plane, a misaligned output, a strided transposed convolution).
+  // N or plane, a misaligned output, a strided transposed convolution); the
+  // general form only.
   constexpr int EBN = Epi::kStageBytes > 0 ? Epi::kStageBytes : 1;
   // the row terms sit past the stage buffers, or (when both do not fit the
   // LDS) at the end of them, written once every load has landed
@@ -512,7 +528,7 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
   const bool zaligned = ((uintptr_t)out.y % 16) == 0;
   if constexpr (Epi::kStageBytes > 0) smode = zaligned && epi.staged_ok() ? 1 : 0;
   if constexpr (kWide) if (smode == 0 && zaligned && epi.staged_wide_ok()) smode = 2;
-  const bool ragged = smode == 0;
+  const bool ragged = Epi::kGeneral && smode == 0;
   if constexpr (Epi::kStageBytes > 0) if (ragged && out.stage && epi.out_bytes() == EBN) smode = 1;
   if constexpr (kWide) if (ragged && out.stage && epi.out_bytes() == 4) smode = 2;
   const bool staged = smode != 0;
@@ -692,7 +708,8 @@ __device__ __forceinline__ void tile_epilogue(const Epi& epi, A (&acc)[Tl::TP][T
     }
   };
   auto flush_any = [&](auto ebc) __attribute__((always_inline)) {
-    if (__builtin_expect(!ragged, 1)) flush(ebc);   // (the common path stays contiguous)
+    if constexpr (!Epi::kGeneral) flush(ebc);
+    else if (__builtin_expect(!ragged, 1)) flush(ebc);   // (the common path stays contiguous)
     else if (out.vec) flush_ragged(ebc, std::integral_constant<int, 4>{});
     else flush_ragged(ebc, std::integral_constant<int, 1>{});
   };
@@ -908,6 +925,7 @@ mfma_gemm_kernel(const LX lx, const LY ly, const Epi epi, int nP, int nQ, int kc
 template <class T> struct PartialEpi {
   T* ws;
   int P, Pp, Q;
+  static constexpr bool kGeneral = false;
   static constexpr bool kHasSimple = false;   // (simple() / finish_simple() are never called)
   static constexpr bool kSimpleTable = false;
   __device__ __forceinline__ int simple(int) const { return 0; }
@@ -921,8 +939,8 @@ template <class T> struct PartialEpi {
   __device__ __forceinline__ void load_i(PreI&, int) const {}
   __device__ __forceinline__ void load_j(PreJ&, int) const {}
   __device__ __forceinline__ int out_bytes() const { return 4; }
-  __device__ __forceinline__ OutAddr addr() const {
-    OutAddr o{};
+  __device__ __forceinline__ PlainAddr addr() const {
+    PlainAddr o{};
     o.y = reinterpret_cast<char*>(ws + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * Q * Pp);
     o.si = 1; o.sj = Pp; o.bstride = 0; o.ohw = 1; o.P = P; o.Q = Q; o.vec = 1;
     return o;
@@ -943,9 +961,9 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const T* __restrict__
   const int groups = Pp / 4;
   const int64_t n = (int64_t)groups * Q;
   const int64_t slice = (int64_t)Q * Pp;   // elements per K slice
-  OutAddr out = epi.addr();
+  auto out = epi.addr();
   out.y += out.slice_offset();
-  ws += (int64_t)blockIdx.z * splits * slice;
+  if constexpr (Epi::kGeneral) ws += (int64_t)blockIdx.z * splits * slice;
   for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n; g += (int64_t)gridDim.x * 256) {
     // n < 2^31 for every workspace the host sizes, so the index split is 32-bit
     const int gi = (int)g;

@@ -1086,6 +1086,38 @@ def test_ragged_output_rows_equal_aligned_ones(torch, ctx, dt, tile):
     assert bool((odd[:, 0] == 7).all()) and bool((odd[:, 1 + n:] == 7).all())
 
 
+@pytest.mark.parametrize("tile", [0, 1, 8, 9, 12])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16", "u8"])
+@pytest.mark.parametrize("group", [1, 2])
+def test_nhwc_outputs_of_either_epilogue(torch, ctx, dt, tile, group):
+    """NHWC outputs at a base one element off (the general epilogue) hold the
+    same bits as aligned ones (the plain one), two groups included."""
+    from oxionnx_amd import _lib as L
+    rng = np.random.default_rng(tile + group)
+    cin, cout, h = 32, 36, 11
+    if dt == "u8":
+        x = _dev(torch, rng.integers(0, 256, (2, cin * group, h, h)).astype(np.uint8))
+        w = ctx.weight_qconv(rng.integers(-127, 128, (cout * group, cin, 3, 3)).astype(np.int8), zp=0, scale=0.01)
+        call = lambda out: ctx.qconv2d(x, w, x_zp=128, out_kind=L.QOUT_U8, x_scale=0.02, y_scale=0.05, y_zp=128,   # noqa: E731
+                                       pads=(1, 1, 1, 1), group=group, out_layout=L.NHWC, out=out)
+    else:
+        tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+        x = _dev(torch, rng.uniform(-1, 1, (2, cin * group, h, h)).astype(np.float32)).to(tdt)
+        w = ctx.weight_conv(rng.normal(0, 0.1, (cout * group, cin, 3, 3)).astype(np.float32), dtype=ldt)
+        call = lambda out: ctx.conv2d(x, w, pads=(1, 1, 1, 1), group=group, out_layout=L.NHWC, out=out)   # noqa: E731
+    ctx.set_tile(tile)
+    try:
+        want = call(None)
+        buf = torch.full((want.numel() + 2,), 7, dtype=want.dtype, device="cuda")
+        got = buf[1:-1].view(want.shape)
+        call(got)
+    finally:
+        ctx.set_tile(0)
+    c = cout * group
+    assert torch.equal(got[..., :c], want[..., :c]) and bool((want[..., :c] != 0).any())
+    assert buf[0] == 7 and buf[-1] == 7 and bool((got[..., c:] == 7).all())
+
+
 # one launch for every image (at least one 64-row tile a phase and image),
 # with and without K slices; (9, 7) is one row short of a tile
 @pytest.mark.parametrize("xs,cout,launches", [((3, 264, 9, 10), 37, 1), ((2, 264, 8, 8), 70, 1), ((3, 40, 11, 13), 5, 1),
