@@ -1031,13 +1031,14 @@ hipError_t run_conv_fewco(int dtype, const void* x, int pitch, const void* w, co
 // A block a CU and one wave a SIMD leave the LDS reads before each MFMA
 // exposed: 64 TFLOP/s there, 41 % of the f32 rate.  The loads go through buffer resources from per-thread
 // offsets formed once; elements outside the image, the channels or the filter
-// read zero through the range check, so the loop has no branch.  k runs
+// read zero through the range check, so the loop has no branch.  (FAR: images
+// or filters past the 31-bit offsets are read through plain pointers.)  k runs
 // (tap, channel): MFMA step j covers k = 2j, 2j + 1, one tap and channels
 // 2j % 8 + {0, 1}, so both operands' addresses are a per-lane base plus a
 // compile-time offset.
 constexpr int kF32Seg = 64, kF32Co = 64, kF32Cs = 8;
 
-template <int KH, int KW, bool MAPPED>
+template <int KH, int KW, bool MAPPED, bool FAR>
 __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ bias, float* __restrict__ y,
                                                             DirectConvArgs a) {
@@ -1061,8 +1062,12 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
   const __amdgpu_buffer_rsrc_t rf =
       __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)co0 * a.ldw), (short)0, 0x7fffffff, 0x00020000);
   // this thread's patch elements and filter chunks of a slab: byte offsets at
-  // slab 0 and the channel (of a chunk: its first) within the slab
-  int poff[NP], pc[NP], foff[NF], fc[NF];
+  // slab 0 (kOob: none) and the channel (of a chunk: its first) within the slab
+  using Off = std::conditional_t<FAR, int64_t, int>;
+  constexpr Off kOob = FAR ? (Off)-1 : (Off)kOobOffset;
+  const float* const wn = w + (int64_t)co0 * a.ldw;
+  Off poff[NP], foff[NF];
+  int pc[NP], fc[NF];
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
     const int i = t + u * 256;
@@ -1078,28 +1083,39 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
       ix = pad_map(ix, a.pl, a.W, a.pad_mode);
     }
     pc[u] = c;
-    poff[u] = ok ? (int)((((int64_t)c * a.H + iy) * a.W + ix) * 4) : kOobOffset;
+    poff[u] = ok ? (Off)((((int64_t)c * a.H + iy) * a.W + ix) * 4) : kOob;
   }
 #pragma unroll
   for (int u = 0; u < NF; ++u) {
     const int i = t + u * 256;        // (co, tap, half)
     const int h = i & 1, r = i >> 1, tap = r % TAPS, co = r / TAPS;
     fc[u] = 4 * h;
-    foff[u] = i < kF32Co * TAPS * 2 && co0 + co < a.cout ? (int)(((int64_t)co * a.ldw + (int64_t)tap * a.cpg + 4 * h) * 4)
-                                                         : kOobOffset;
+    foff[u] = i < kF32Co * TAPS * 2 && co0 + co < a.cout ? (Off)(((int64_t)co * a.ldw + (int64_t)tap * a.cpg + 4 * h) * 4)
+                                                         : kOob;
   }
   struct Slab { float p[NP]; u32x4 f[NF]; };
   auto load = [&](Slab& d, int sl) __attribute__((always_inline)) {
     const int c0 = sl * kF32Cs, left = a.C - c0, leftf = a.cpg - c0;   // (<= 0 past the last slab: all read zero)
+    if constexpr (FAR) {
+      const char* xs = reinterpret_cast<const char*>(xn) + (int64_t)c0 * a.H * a.W * 4;
+      const char* ws = reinterpret_cast<const char*>(wn) + (int64_t)c0 * 4;
+#pragma unroll
+      for (int u = 0; u < NP; ++u)
+        d.p[u] = poff[u] != kOob && pc[u] < left ? *reinterpret_cast<const float*>(xs + poff[u]) : 0.0f;
+#pragma unroll
+      for (int u = 0; u < NF; ++u)
+        d.f[u] = foff[u] != kOob && fc[u] < leftf ? *reinterpret_cast<const u32x4*>(ws + foff[u]) : u32x4{0u, 0u, 0u, 0u};
+      return;
+    }
     const int so = __builtin_amdgcn_readfirstlane(left > 0 ? (int)((int64_t)c0 * a.H * a.W * 4) : 0);
     const int sf = __builtin_amdgcn_readfirstlane(leftf > 0 ? c0 * 4 : 0);
 #pragma unroll
     for (int u = 0; u < NP; ++u)
-      d.p[u] = lane_f32((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rx, pc[u] < left ? poff[u] : kOobOffset, so, 0));
+      d.p[u] = lane_f32((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rx, pc[u] < left ? (int)poff[u] : kOobOffset, so, 0));
 #pragma unroll
     for (int u = 0; u < NF; ++u)
       d.f[u] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rf, fc[u] < leftf ? foff[u] : kOobOffset, sf, 0));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rf, fc[u] < leftf ? (int)foff[u] : kOobOffset, sf, 0));
   };
   auto store = [&](const Slab& s, int b) __attribute__((always_inline)) {
     float* pd = lds[b];
@@ -1185,9 +1201,7 @@ __global__ void __launch_bounds__(256) conv_nchw_f32_kernel(const float* __restr
 
 bool conv_nchw_f32_supported(const DirectConvArgs& a) {
   return a.KH == a.KW && (a.KH == 3 || (a.KH == 1 && a.pad_mode == 0)) && a.sh == 1 && a.sw == 1 && a.dh == 1 && a.dw == 1 &&
-         !a.nhwc_out && a.cpg % 4 == 0 && a.ldw % 4 == 0 &&
-         // 32-bit buffer offsets
-         ((int64_t)a.C + kF32Cs) * a.H * a.W * 4 < 0x7fffffff && (int64_t)kF32Co * a.ldw * 4 < 0x7fffffff;
+         !a.nhwc_out && a.cpg % 4 == 0 && a.ldw % 4 == 0;
 }
 
 hipError_t run_conv_nchw_f32(const float* x, const float* w, const float* bias, float* y, const DirectConvArgs& a,
@@ -1197,12 +1211,20 @@ hipError_t run_conv_nchw_f32(const float* x, const float* w, const float* bias, 
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks, (unsigned)((a.cout + kF32Co - 1) / kF32Co));
-  if (a.KH == 3 && a.pad_mode != 0)
-    hipLaunchKernelGGL((conv_nchw_f32_kernel<3, 3, true>), grid, dim3(256), 0, st, x, w, bias, y, a);
-  else if (a.KH == 3)
-    hipLaunchKernelGGL((conv_nchw_f32_kernel<3, 3, false>), grid, dim3(256), 0, st, x, w, bias, y, a);
+  auto go = [&](auto far) {
+    constexpr bool FAR = decltype(far)::value;
+    if (a.KH == 3 && a.pad_mode != 0)
+      hipLaunchKernelGGL((conv_nchw_f32_kernel<3, 3, true, FAR>), grid, dim3(256), 0, st, x, w, bias, y, a);
+    else if (a.KH == 3)
+      hipLaunchKernelGGL((conv_nchw_f32_kernel<3, 3, false, FAR>), grid, dim3(256), 0, st, x, w, bias, y, a);
+    else
+      hipLaunchKernelGGL((conv_nchw_f32_kernel<1, 1, false, FAR>), grid, dim3(256), 0, st, x, w, bias, y, a);
+  };
+  // 31-bit offsets into an image and into a block's 64 filters, else FAR
+  if (((int64_t)a.C + kF32Cs) * a.H * a.W * 4 < 0x7fffffff && (int64_t)kF32Co * a.ldw * 4 < 0x7fffffff)
+    go(std::false_type{});
   else
-    hipLaunchKernelGGL((conv_nchw_f32_kernel<1, 1, false>), grid, dim3(256), 0, st, x, w, bias, y, a);
+    go(std::true_type{});
   return hipGetLastError();
 }
 

@@ -94,3 +94,35 @@ def test_noalloc_halo_without_room(torch, ctx, xs, cout):
     torch.cuda.synchronize()
     assert ctx.counters()["device_allocs"] == 0
     assert torch.equal(got, want)
+
+
+# an image of 2 GiB, past the in-place f32 kernel's 31-bit offsets: the same
+# sums as the bands of rows that it is cut into here, and no staged copy
+@pytest.mark.parametrize("k,mode", [(3, "zeros"), (1, "zeros"), (3, "reflect")])
+def test_noalloc_of_an_image_past_31_bits(torch, ctx, k, mode):
+    from oxionnx_amd import _lib as L
+    c, cout, h, w = 64, 12, 2900, 2901
+    x = torch.empty((1, c, h, w), device="cuda")
+    x.uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(k))
+    rng = np.random.default_rng(k)
+    wt = ctx.weight_conv(rng.normal(0, 0.1, (cout, c, k, k)).astype(np.float32))
+    p = k // 2
+    y = torch.full((1, cout, h, w), float("nan"), device="cuda")
+
+    def call(src, dst, rows, pt, pb):   # (the descriptor takes the pad mode, which conv2d() does not)
+        d = L.ConvDesc(1, c, rows, w, cout, k, k, 1, 1, 1, 1, 1, pt, p, pb, p, L.F32, L.NCHW, L.NCHW, L.ACT_NONE, 0.0, 0.0,
+                       L.PAD_REFLECT if mode == "reflect" else L.PAD_ZEROS)
+        L.check(L.lib().ohip_conv2d_noalloc(ctx.h, ctypes.byref(d), src.data_ptr(), wt.handle, None, dst.data_ptr()))
+
+    torch.cuda.synchronize()
+    ctx.reset_counters()
+    call(x, y, h, p, p)
+    torch.cuda.synchronize()
+    assert ctx.counters()["device_allocs"] == 0
+    for r0, r1 in ((0, 64), (1400, 1464), (h - 64, h)):   # output rows; the bands' inner edges have no pad
+        a, b = max(r0 - p, 0), min(r1 + p, h)
+        pt, pb = (p if a == 0 else 0), (p if b == h else 0)
+        part = torch.empty((1, cout, b - a + pt + pb - 2 * p, w), device="cuda")
+        call(x[:, :, a:b].contiguous(), part, b - a, pt, pb)
+        assert torch.equal(y[:, :, r0:r1], part)
+    assert not bool(torch.isnan(y).any())
