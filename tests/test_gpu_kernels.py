@@ -211,11 +211,10 @@ GROUP_CASES = [
     ((2, 48, 6, 6), (48, 16, 1, 1), 3, (1, 1), (0, 0, 0, 0), (1, 1)),       # 1x1, aligned groups
     ((2, 8, 11, 13), (8, 1, 3, 3), 8, (1, 1), (1, 1, 1, 1), (1, 1)),        # depthwise
     ((1, 6, 9, 9), (12, 1, 5, 5), 6, (2, 2), (2, 1, 2, 1), (1, 1)),         # depthwise, multiplier 2
-    # depthwise 3x3 on the band kernel (from 2^18 outputs): bands of 56x56
-    # planes, stride 2 with odd extents, uneven pads, a valid conv, 2000-wide
-    # rows (four-row windows); the same geometries below 2^18 outputs take
-    # the one-thread-per-output kernel; rows of whole 16-byte chunks are
-    # staged by chunk loads
+    # depthwise 3x3 of 2^18 outputs: 56x56 planes, stride 2 with odd extents,
+    # uneven pads, a valid conv, 2000-wide rows; the strip kernel takes all
+    # but the one with a pad of two (the band kernel, staged by chunk loads;
+    # more of those in test_depthwise_3x3_bands)
     ((2, 96, 56, 56), (96, 1, 3, 3), 96, (1, 1), (1, 1, 1, 1), (1, 1)),
     ((1, 288, 115, 63), (288, 1, 3, 3), 288, (2, 2), (1, 1, 1, 1), (1, 1)),
     ((1, 256, 66, 129), (256, 1, 3, 3), 256, (2, 2), (0, 1, 1, 0), (1, 1)),
@@ -259,8 +258,7 @@ def test_grouped_conv_matches_oracle(torch, ctx, case, dt):
         assert _rel_err(got, want) <= HALF_TOL
 
 
-# bf16 depthwise 3x3 on both sides of the band kernel's 2^18-output gate,
-# against torch's f32 conv of the same bf16-rounded operands (the oracle has
+# bf16 depthwise 3x3 (the strip kernel) on both sides of 2^18 outputs, against torch's f32 conv of the same bf16-rounded operands (the oracle has
 # no bf16 conv): (x shape, stride, pads [t, l, b, r]).
 DW_BF16_CASES = [((1, 96, 76, 76), 1, (1, 1, 1, 1)), ((1, 288, 115, 63), 2, (1, 1, 1, 1)),
                  ((2, 8, 12, 10), 1, (0, 1, 1, 0))]
@@ -1423,3 +1421,102 @@ def test_depthwise_3x3_strips(torch, ctx, h, w, s, pads, dt):
     want = want.clamp(-0.5, 0.5)
     assert y.shape == want.shape
     assert torch.allclose(y.double(), want, rtol=0, atol=1e-5 if dt == "f32" else 8e-3, equal_nan=True)
+
+
+def _dw3_want(torch, x, k, b, s, pads):
+    """torch's f32 depthwise convolution of the same rounded operands."""
+    xp = torch.nn.functional.pad(x.float(), (pads[1], pads[3], pads[0], pads[2]))
+    return torch.nn.functional.conv2d(xp, k.float(), b.float(), stride=s, groups=x.shape[1])
+
+
+# the strip kernel's wide strips (from 2^17 of them) and its two rows a thread
+# (from 2^19 threads): 5000 and 20000 planes of 7 output rows (a cut last group)
+# by 30 (a last strip that overlaps), 17-element runs at stride 2
+@pytest.mark.parametrize("n", [50, 200])
+@pytest.mark.parametrize("s", [1, 2])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_depthwise_3x3_strips_of_many_planes(torch, ctx, n, s, dt):
+    from oxionnx_amd import _lib as L
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    g = torch.Generator(device="cuda").manual_seed(n + s)
+    h, w = (7, 30) if s == 1 else (13, 59)
+    x = (torch.rand((n, 100, h, w), generator=g, device="cuda") * 2 - 1).to(tdt)
+    k = (torch.randn((100, 1, 3, 3), generator=g, device="cuda") * 0.3).to(tdt)
+    b = (torch.randn(100, generator=g, device="cuda") * 0.1).to(tdt)
+    y = ctx.conv2d(x, ctx.weight_conv(k.float().cpu().numpy(), dtype=ldt), b, strides=(s, s), pads=(1, 1, 1, 1), group=100)
+    want = _dw3_want(torch, x, k, b, s, (1, 1, 1, 1))
+    assert y.shape == want.shape == (n, 100, 7, 30)
+    assert float((y.float() - want).abs().max() / want.abs().max()) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+# the band kernel: pads of two, from 2^18 outputs (x shape, stride, pads)
+@pytest.mark.parametrize("xs,s,pads", [((2, 96, 56, 56), 1, (2, 2, 2, 2)), ((1, 288, 115, 63), 2, (2, 2, 1, 1)),
+                                       ((1, 16, 17, 2000), 1, (1, 2, 1, 2)), ((1, 96, 76, 75), 1, (0, 2, 1, 0))], ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_depthwise_3x3_bands(torch, ctx, xs, s, pads, dt):
+    from oxionnx_amd import _lib as L
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    g = torch.Generator(device="cuda").manual_seed(xs[1] + s)
+    c = xs[1]
+    x = (torch.rand(xs, generator=g, device="cuda") * 2 - 1).to(tdt)
+    k = (torch.randn((c, 1, 3, 3), generator=g, device="cuda") * 0.3).to(tdt)
+    b = (torch.randn(c, generator=g, device="cuda") * 0.1).to(tdt)
+    y = ctx.conv2d(x, ctx.weight_conv(k.float().cpu().numpy(), dtype=ldt), b, strides=(s, s), pads=pads, group=c)
+    want = _dw3_want(torch, x, k, b, s, pads)
+    assert y.shape == want.shape and y.numel() >= 1 << 18
+    assert float((y.float() - want).abs().max() / want.abs().max()) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+# GEMV over long rows (the skinny kernel's 16-row blocks would leave CUs idle):
+# one and two weight rows a block, an odd last one, and the activation loads
+# in two halves (16 bits, 6 to 8 rows, one weight row a block)
+@pytest.mark.parametrize("dt,n", [("f16", 640), ("f16", 769), ("f16", 1025), ("bf16", 640), ("bf16", 769), ("f32", 511),
+                                  ("f32", 513)])
+def test_gemv_of_several_rows(torch, ctx, dt, n):
+    from oxionnx_amd import _lib as L
+    k = 12504 if dt == "f32" else 25008   # 3126 chunks: no whole number of the block's rounds
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    g = torch.Generator(device="cuda").manual_seed(n)
+    b = (torch.randn((k, n), generator=g, device="cuda") * k ** -0.5).to(tdt)
+    w = ctx.weight_gemm(b.float().cpu().numpy(), dtype=ldt)
+    for m in range(2, 9):
+        a = (torch.rand((m, k), generator=g, device="cuda") * 2 - 1).to(tdt)
+        want = (a.double() @ b.double()).cpu().numpy()
+        assert _rel_err(ctx.gemm(a, w).double().cpu().numpy(), want) <= (F32_TOL if dt == "f32" else HALF_TOL), m
+
+
+@pytest.mark.parametrize("k,n", [(7, 16), (777, 130), (5001, 40)])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_gemm_of_one_misaligned_row(torch, ctx, k, n, dt):
+    from oxionnx_amd import _lib as L
+    tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    rng = np.random.default_rng(k)
+    a = _dev(torch, rng.uniform(-1, 1, (1, k + 1)).astype(np.float32)).to(tdt)[:, 1:]
+    b = _dev(torch, rng.normal(0, k ** -0.5, (k, n)).astype(np.float32)).to(tdt)
+    got = ctx.gemm(a, ctx.weight_gemm(b.float().cpu().numpy(), dtype=ldt))
+    assert _rel_err(got.double().cpu().numpy(), (a.double() @ b.double()).cpu().numpy()) <= (F32_TOL if dt == "f32" else HALF_TOL)
+
+
+# several images a tile, NCHW out: planes of whole 16-byte chunks that are no
+# multiple of the tile (12x12 bytes), and of four elements (14x14 of 16 bits)
+@pytest.mark.parametrize("dt,hw", [("u8", 12), ("f16", 14), ("bf16", 14), ("f16", 12)])
+def test_images_that_share_an_output_tile(torch, ctx, dt, hw):
+    from oxionnx_amd import _lib as L
+    rng = np.random.default_rng(hw)
+    shape, ws = (5, 48, hw, hw), (37, 48, 3, 3)
+    if dt == "u8":
+        x = rng.integers(0, 256, shape).astype(np.uint8)
+        w = rng.integers(-127, 128, ws).astype(np.int8)
+        call = lambda v: ctx.qconv2d(v, wt, x_zp=128, out_kind=L.QOUT_U8, x_scale=0.02, y_scale=0.9, y_zp=128,   # noqa: E731
+                                     pads=(1, 1, 1, 1))
+        wt = ctx.weight_qconv(w, zp=0, scale=0.01)
+        want = O.qlinear_conv(x, 0.02, 128, w, np.full(37, 0.01, np.float32), np.zeros(37, np.int32), 0.9, 128,
+                              sat_range=(0, 255), pads=(1, 1, 1, 1))
+        np.testing.assert_array_equal(call(_dev(torch, x)).cpu().numpy().astype(np.float32), want)
+        return
+    tdt, ldt = {"f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
+    x = _dev(torch, rng.uniform(-1, 1, shape).astype(np.float32)).to(tdt)
+    w = _dev(torch, rng.normal(0, 0.05, ws).astype(np.float32)).to(tdt)
+    y = ctx.conv2d(x, ctx.weight_conv(w.float().cpu().numpy(), dtype=ldt), pads=(1, 1, 1, 1))
+    want = torch.nn.functional.conv2d(x.double().cpu(), w.double().cpu(), padding=1).numpy()
+    assert _rel_err(y.double().cpu().numpy(), want) <= HALF_TOL
