@@ -1426,7 +1426,7 @@ static bool staged_f32_wins(ohip_ctx* ctx, const ohip_conv_desc* d, int64_t rows
   const float n = std::ceil(blocks / 256.0f), slabs = (float)((d->c + 7) / 8);
   const float in_place = 3.3f + slabs * (n <= 1.0f ? (k3 ? 1.75f : .31f) : n * (k3 ? 1.65f : .33f));
   const float staging = 2.6f + (float)staged * 2e-6f / 2.5f;
-  return 1.15f * (sc.us + 3.1f + staging) < in_place;
+  return 1.15f * (sc.us + (sc.splits > 1 ? 4.4f : 3.1f) + staging) < in_place;
 }
 
 static int conv2d_impl(ohip_ctx* ctx, const ohip_conv_desc* d, const void* x, const ohip_weight* w, const void* bias,

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 namespace ohip {
 
@@ -45,14 +46,20 @@ struct ReduceCost {
 enum class PlanKind { Dense, DenseF32, Conv };   // f16 / bf16 / int8 rows; f32 of any loader; im2col rows
 
 // The tile and the split of a contraction P x Q (x batch) over kc 16-byte
-// chunks, by the cost of every candidate.  The constants are a least-squares
-// fit to 178 shapes (M 12-4096, K 64-16384, N 64-11008; 1x1-5x5 convolutions
-// of 7-112 pixels; f16, f32, int8) timed on every tile and on 2-16 slices, graph
-// replay: the plan is within 1 % of the fastest candidate in the geometric
-// mean (worst 1.12x), where the rules it replaces, thresholds on the number
-// of blocks, were 8.8 % (dense), 11 % (f32) and 5 % (convolutions) from it,
-// up to 1.6x: f16 1024x1024x768 13.7 -> 9.0 us (split, now unsplit),
-// 1500x1024x2048 18.0 -> 12.7, 838x2688x2880 37 -> 24.
+// chunks, by the cost of every candidate.  The tiles' constants are a
+// least-squares fit to 178 shapes (M 12-4096, K 64-16384, N 64-11008; 1x1-5x5
+// convolutions of 7-112 pixels; f16, f32, int8) timed on every tile, graph
+// replay, and so are the slices of the 16-bit and int8 convolutions (their
+// reduction's launch also costs the host about 1.5 us, which is in its fixed
+// term whether or not a host waits: a capture has to plan as the eager call
+// before it did, for the same scratch and the same bits).  The slices of the
+// other kinds are fitted to 104 products of 33-600 rows timed on 2-16 slices,
+// eager and by replay (their mean), by the loss of the choice: 0.2 % in the
+// mean for f32 (1.8 % at most), 0.9 % for f16 and int8 (7 %).  Every count up
+// to ten is a candidate there: 48 blocks of f32 200x2048x768 fill a round with
+// five slices (16.7 us; four 18.3, six 19.5).  Against rules on the number of
+// blocks: f16 1024x1024x768 13.7 -> 9.0 us (split, now unsplit), 1500x1024x2048
+// 18.0 -> 12.7, 838x2688x2880 37 -> 24.
 // Grids of a round of 256x256 tiles and a long K take tile 16 outright: its
 // advantage there is the clock and the cache, which the stages' cost does
 // not show (4096x4096x11008 f16 291 us against 324 on tiles 3, 4 and 18).
@@ -77,10 +84,8 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   static constexpr TileCost kConv[] = {{1, 64, 64, 4, .522f, .234f, 1.17f},   {9, 64, 64, 2, .386f, .254f, 1.17f},
                                        {8, 128, 128, 2, .633f, .403f, 1.56f}, {12, 128, 128, 1, .510f, .510f, 2.15f},
                                        {3, 256, 128, 1, .708f, .708f, 4.0f},  {4, 128, 256, 1, .708f, .708f, 4.0f}};
-  // (+ 1.5: a launch more also costs the host about 2 us, which small eager
-  // calls wait for: 5x960x1920 int8 pair 16.5 us, 18.8 with its second split)
-  const ReduceCost red = kind == PlanKind::Dense      ? ReduceCost{1.82f + 1.5f, .367f, .146f}
-                         : kind == PlanKind::DenseF32 ? ReduceCost{1.81f + 1.5f, .229f, .122f}
+  const ReduceCost red = kind == PlanKind::Dense      ? ReduceCost{1.5f, .35f, .18f}
+                         : kind == PlanKind::DenseF32 ? ReduceCost{2.0f, .50f, .03f}
                                                       : ReduceCost{1.21f + 1.5f, .321f, .121f};
   const TileCost* tab = kind == PlanKind::Dense ? kDense : kind == PlanKind::DenseF32 ? kF32 : kConv;
   const int ntab = kind == PlanKind::Dense      ? (int)(sizeof(kDense) / sizeof(TileCost))
@@ -109,7 +114,7 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   };
   auto time = [&](const TileCost& t, int64_t nb, int64_t stages) {
     const uint32_t ncu = (uint32_t)std::min<int64_t>((nb + 255) >> 8, 1 << 24), res = (uint32_t)t.res;
-    const uint32_t q = ncu / res, rem = ncu - q * res;
+    const uint32_t q = ncu >> (res >> 1), rem = ncu & (res - 1);   // (res is 1, 2 or 4)
     return t.fix * (float)(q + (rem ? 1 : 0)) +
            (float)stages * ((float)q * std::max(t.lat, (float)t.res * t.bw) + (rem ? std::max(t.lat, (float)rem * t.bw) : 0.0f));
   };
@@ -125,14 +130,27 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     const float c = time(t, nb, nk);
     if (c < cost) { cost = c; best = {1, t.id}; }
     if (!may_split || (t.id != 9 && t.id != 8)) continue;
-    for (const int most : {2, 3, 4, 6, 8, 12, 16}) {
+    const float mb = (float)P * (float)Q * (float)batch * 4e-6f;
+    // (each count a constant: small eager calls wait for this)
+    auto slices = [&](auto count) {
+      constexpr uint32_t most = decltype(count)::value;
       const uint32_t per = ((uint32_t)nk + most - 1) / most;
-      if (per < 2) break;
-      const int s = filled(most);
-      const float cs = time(t, nb * s, per) + red.fix + red.per_slice * (float)s +
-                       red.per_mb * (float)P * (float)Q * (float)batch * (float)s * 4e-6f;
+      if (per < 2) return false;
+      const int s = per * (most - 1) < (uint32_t)nk ? (int)most : filled(most);
+      const float cs = time(t, nb * s, per) + red.fix + red.per_slice * (float)s + red.per_mb * mb * (float)s;
       if (cs < cost) { cost = cs; best = {s, t.id == 9 ? 10 : 11}; }
-    }
+      return true;
+    };
+    auto all = [&](auto... count) { (void)(slices(count) && ...); };
+    using std::integral_constant;
+    if (kind == PlanKind::Conv)
+      all(integral_constant<int, 2>{}, integral_constant<int, 3>{}, integral_constant<int, 4>{}, integral_constant<int, 6>{},
+          integral_constant<int, 8>{}, integral_constant<int, 12>{}, integral_constant<int, 16>{});
+    else
+      all(integral_constant<int, 2>{}, integral_constant<int, 3>{}, integral_constant<int, 4>{}, integral_constant<int, 5>{},
+          integral_constant<int, 6>{}, integral_constant<int, 7>{}, integral_constant<int, 8>{}, integral_constant<int, 9>{},
+          integral_constant<int, 10>{}, integral_constant<int, 12>{}, integral_constant<int, 14>{},
+          integral_constant<int, 16>{});
   }
   if (best.splits == 1 && kind == PlanKind::Dense && !wide_out) {
     const TileCost& t = kDense[ntab - 1];
@@ -170,7 +188,7 @@ inline bool skinny_wins(bool f32, int64_t m, int64_t n, int64_t kc, bool pack, c
   const float skinny =
       std::max(step * steps, mb / rate) + acts * (f32 ? .01f : .05f) + (m > 16 ? mb * (f32 ? .2f : .12f) : 0.0f);
   const float other = m <= kMaxGemvM ? mb / 7.0f + rows * (.33f + (f32 ? .02f : m <= 2 ? .022f : .04f) * mb)
-                                     : engine.us + (engine.splits == 1 ? 2.2f : .2f);
+                                     : engine.us + (engine.splits == 1 ? 2.2f : 1.5f);
   return skinny < other + (pack ? 2.5f : 0.0f);
 }
 

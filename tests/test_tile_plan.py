@@ -89,3 +89,24 @@ def test_few_rows_take_the_faster_kernel(lib, case):
     dt, m, k, n, skinny, other = case
     per = 4 if dt == "f32" else 8
     assert bool(lib.skinny(int(dt == "f32"), m, n, -(-k // per), int(k % per != 0))) == (skinny < other)
+
+
+# (kind, elements a chunk, rows, K, N): us by K slices (1: the fastest tile unsplit)
+SPLITS = [((1, 4, 128, 768, 3072), {1: 20.2, 2: 15.6, 3: 18.0, 4: 16.8, 5: 16.7, 6: 20.1, 8: 18.8}),
+          ((1, 4, 128, 1024, 4096), {1: 25.3, 2: 19.4, 3: 22.4, 4: 21.5, 5: 24.4, 8: 23.1}),
+          ((1, 4, 200, 2048, 768), {1: 46.6, 3: 21.8, 4: 18.3, 5: 16.7, 6: 19.5, 7: 20.1, 8: 18.5, 10: 17.9}),
+          ((1, 4, 527, 2064, 662), {1: 49.0, 2: 30.0, 3: 32.2, 4: 28.0, 5: 25.2, 6: 29.8, 8: 29.2}),
+          ((1, 4, 132, 2818, 766), {1: 68.0, 4: 26.2, 5: 23.4, 6: 21.7, 7: 20.9, 8: 23.0, 9: 24.6, 12: 23.4}),
+          ((1, 4, 156, 6864, 1074), {1: 149.6, 5: 37.4, 8: 39.0, 9: 36.8, 10: 35.0, 12: 42.9}),
+          ((1, 4, 256, 768, 3072), {1: 21.0, 2: 23.2, 3: 26.8, 4: 23.5, 5: 24.8}),
+          ((0, 8, 128, 768, 3072), {1: 7.4, 2: 9.0, 3: 10.3, 4: 10.8}),
+          ((0, 8, 128, 8192, 4096), {1: 57.9, 3: 26.2, 4: 23.7, 5: 28.2, 8: 28.3}),
+          ((0, 16, 300, 2048, 512), {1: 10.1, 2: 9.6, 3: 9.2, 4: 8.8, 5: 9.5, 6: 9.5, 8: 10.3}),
+          ((0, 16, 206, 1931, 159), {1: 13.1, 2: 12.0, 3: 11.4, 4: 10.8, 5: 11.3, 6: 11.1, 8: 10.9, 12: 11.5})]
+
+
+@pytest.mark.parametrize("shape,us", SPLITS, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_k_slices_near_the_fastest_measured(plan, shape, us):
+    kind, per, m, k, n = shape
+    splits, _, _ = plan(kind, n, m, -(-k // per))
+    assert splits in us and us[splits] <= 1.05 * min(us.values()), (splits, us)
