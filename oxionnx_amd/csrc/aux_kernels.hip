@@ -106,11 +106,11 @@ template <> struct Vec16<__bf16> {
 // registers and LDS in a fixed order (deterministic), and the first NR * M
 // threads run the epilogue for the outputs of those rows.  Two rows a block
 // share the activation chunks, which the blocks read from L2 (M times the
-// weight's bytes in all with one row a block): 5x4096x4096 f16 23.4 -> 18.9
-// us, 2x4096x1024 f32 6.3 -> 5.2; with fewer weight rows they leave CUs idle
+// weight's bytes in all with one row a block): 2x4096x1024 f32 6.3 -> 5.2 us;
+// with fewer weight rows they leave CUs idle
 // (5x25088x512 f16 11.3, 13.0 with two).  Products are summed by fused
 // multiply-adds (that shape 13.4 us with a multiply and an add).
-template <class T, int M, int NR>
+template <class T, int M, int NR, bool SERIAL = false>
 __global__ void __launch_bounds__(512, sizeof(T) == 2 && NR == 1 ? 6 : 1)
 gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, int64_t ldw, int kc, int N,
                 FloatEpi<T> epi) {
@@ -134,9 +134,10 @@ gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, i
   constexpr int U = (sizeof(T) == 4 ? 16 : 8) / NR;
   // activation loads issued together: all M, or half of them where all would
   // leave a CU two blocks instead of three (8x5952x640 bf16 10.4 -> 9.0 us,
-  // 7x5952x640 f16 10.3 -> 8.1; with three anyway they lose 1-6 %)
+  // 7x5952x640 f16 10.3 -> 8.1; with three anyway they lose 1-6 %).  SERIAL:
+  // as the compiler places them.
   constexpr bool half = sizeof(T) == 2 && NR == 1 && M >= (std::is_same<T, __bf16>::value ? 6 : 7);
-  constexpr int AB = half ? (M + 1) / 2 : M;
+  constexpr int AB = SERIAL ? 1 : half ? (M + 1) / 2 : M;
   for (int c = tid; c < kc; c += U * S) {
     u32x4 wv[U][NR];
 #pragma unroll
@@ -156,7 +157,7 @@ gemv_row_kernel(const T* __restrict__ a, int64_t lda, const T* __restrict__ w, i
 #pragma unroll
           for (int m = m0; m < m0 + AB && m < M; ++m)
             av[m - m0] = reinterpret_cast<const u32x4*>(a + (int64_t)m * lda)[c + u * S];
-          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (!SERIAL) __builtin_amdgcn_sched_barrier(0);
           if (m0 == 0)
 #pragma unroll
             for (int i = 0; i < NR; ++i) Vec16<T>::unpack(wv[u][i], f[i]);
@@ -247,9 +248,19 @@ static hipError_t gemv_t(const GemvArgs& g, const FloatOut& o, hipStream_t st) {
   const bool by_wave = g.kc <= kWaveRowChunks;
   // weight rows from which two a block still fill the chip; earlier where the
   // registers leave a CU three blocks of one row each and those need a second
-  // round (3x5000x1000 bf16 7.7 -> 6.0 us, 6x5200x900 9.6 -> 8.3)
+  // round (3x5000x1000 bf16 7.7 -> 6.0 us, 6x5200x900 9.6 -> 8.3).  In f32 two
+  // from the 512 rows that are one round of one each (2x8192x576 8.6 -> 7.3),
+  // but 512 themselves only over a long K (2x8192x512 6.6 us, 5.5 with one;
+  // 4x25088x512 14.1, 16.7 with one)
   const int m3 = std::is_same<T, __bf16>::value ? 3 : 5;
-  const int two_rows = sizeof(T) == 4 ? 512 : g.M >= m3 ? 769 : 1024;
+  const bool two_rows = sizeof(T) == 4 ? g.N > 512 || (g.N == 512 && g.kc > 2048) : g.N >= (g.M >= m3 ? 769 : 1024);
+  // one weight row a block, more blocks than a round of two a CU (f32, five
+  // activation rows: of one) and a long K: the activations' reads from L2 bound
+  // it, and issued together they gain nothing any more (8x25088x576 bf16 20.2
+  // -> 18.2 us, f16 19.8 -> 18.0, 8x12000x576 f16 11.7, 12.4 serial; f32
+  // 8x25088x300 23.5 -> 21.4, 6x16000x400 14.3 -> 13.5, 7x9000x400 10.0, 10.3
+  // serial, 6x25088x200 10.8, 15.0 serial)
+  const bool serial = sizeof(T) == 2 ? g.N > 512 && g.kc >= 2000 : g.M >= 5 && g.N > 256 && g.kc >= 3000;
   const unsigned wave_blocks = (unsigned)((g.N + 3) / 4);
   switch (g.M) {
 #define OHIP_GEMV_CASE(MM)                                                                                      \
@@ -257,8 +268,11 @@ static hipError_t gemv_t(const GemvArgs& g, const FloatOut& o, hipStream_t st) {
     if (by_wave)                                                                                                \
       hipLaunchKernelGGL((gemv_wave_kernel<T, MM>), dim3(wave_blocks), dim3(256), 0, st, a, g.lda, w, g.ldw, \
                          g.kc, g.N, epi);                                                                       \
-    else if (MM > 1 && g.N >= two_rows)                                                                             \
+    else if (MM > 1 && two_rows)                                                                                    \
       hipLaunchKernelGGL((gemv_row_kernel<T, MM, MM == 1 ? 1 : 2>), dim3((g.N + 1) / 2), dim3(512), 0, st, a, g.lda, w, \
+                         g.ldw, g.kc, g.N, epi);                                                                \
+    else if (MM > 1 && serial)                                                                                  \
+      hipLaunchKernelGGL((gemv_row_kernel<T, MM, 1, (MM > 1)>), dim3(g.N), dim3(512), 0, st, a, g.lda, w, \
                          g.ldw, g.kc, g.N, epi);                                                                \
     else                                                                                                        \
       hipLaunchKernelGGL((gemv_row_kernel<T, MM, 1>), dim3(g.N), dim3(512), 0, st, a, g.lda, w, g.ldw, g.kc, g.N, epi); \

@@ -65,8 +65,10 @@ enum class PlanKind { Dense, DenseF32, Conv };   // f16 / bf16 / int8 rows; f32 
 // not show (4096x4096x11008 f16 291 us against 324 on tiles 3, 4 and 18).
 // A convolution's tile 1 is charged 0.5 us a round above its fit: the fit's
 // replays find every operand in the cache, a forward's convolution does not,
-// and two LDS stages hide less of that than tile 9's four (512 blocks of a
-// generator's 3x3 stride-2 f16 convolution 11.7 us on tile 1, 10.4 on 9).
+// and two LDS stages hide less of that than tile 9's four.  (Seen on 512 blocks
+// of one generator's 3x3 stride-2 f16 convolution: 11.7 us on tile 1, 10.4 on
+// 9.  24 other unsplit convolutions by replay: f16 0-6 % faster on tile 9, int8
+// 3-5 % faster on tile 1, which the charge costs them.)
 // The split is symmetric in P and Q (a convolution splits alike in NCHW and
 // NHWC output), so it is chosen without the one tile that is not square or
 // paired, 18 (whose 4-byte outputs do not fit its stage buffers: wide_out).
@@ -186,8 +188,8 @@ inline bool skinny_wins(bool f32, int64_t m, int64_t n, int64_t kc, bool pack, c
   const float step = f32 ? .29f + .0125f * rows : .25f + .0115f * rows;
   const float rate = f32 ? (steps >= 8.0f ? 5.4f : 4.2f) : steps >= 16.0f ? 6.5f : steps >= 8.0f ? 5.4f : 4.6f;   // MB a us
   const float skinny =
-      std::max(step * steps, mb / rate) + acts * (f32 ? .01f : .05f) + (m > 16 ? mb * (f32 ? .2f : .12f) : 0.0f);
-  const float other = m <= kMaxGemvM ? mb / 7.0f + rows * (.33f + (f32 ? .02f : m <= 2 ? .022f : .04f) * mb)
+      std::max(step * steps, mb / rate) + acts * (f32 ? .01f : m > kMaxGemvM ? .05f : 0.0f) + (m > 16 ? mb * (f32 ? .2f : .12f) : 0.0f);
+  const float other = m <= kMaxGemvM ? mb / 7.0f + rows * (.33f + (f32 ? .02f : m <= 2 ? .018f : .04f) * mb)
                                      : engine.us + (engine.splits == 1 ? 2.2f : 1.5f);
   return skinny < other + (pack ? 2.5f : 0.0f);
 }

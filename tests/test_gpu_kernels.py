@@ -1468,13 +1468,15 @@ def test_depthwise_3x3_bands(torch, ctx, xs, s, pads, dt):
 
 
 # GEMV over long rows (the skinny kernel's 16-row blocks would leave CUs idle):
-# one and two weight rows a block, an odd last one, and the activation loads
-# in two halves (16 bits, 6 to 8 rows, one weight row a block)
-@pytest.mark.parametrize("dt,n", [("f16", 640), ("f16", 769), ("f16", 1025), ("bf16", 640), ("bf16", 769), ("f32", 511),
-                                  ("f32", 513)])
-def test_gemv_of_several_rows(torch, ctx, dt, n):
+# one and two weight rows a block, an odd last one, the activation loads in two
+# halves (16 bits, 6 to 8 rows, one weight row a block) and as they come; no K
+# is a whole number of the block's rounds
+@pytest.mark.parametrize("dt,n,k", [("f16", 640, 15000), ("f16", 640, 25008), ("f16", 769, 25008), ("f16", 1025, 25008),
+                                    ("bf16", 640, 15000), ("bf16", 640, 25008), ("bf16", 769, 25008),
+                                    ("f32", 511, 12504), ("f32", 512, 12504), ("f32", 512, 8192), ("f32", 513, 8192),
+                                    ("f32", 513, 12504), ("f32", 705, 12504)])
+def test_gemv_of_several_rows(torch, ctx, dt, n, k):
     from oxionnx_amd import _lib as L
-    k = 12504 if dt == "f32" else 25008   # 3126 chunks: no whole number of the block's rounds
     tdt, ldt = {"f32": (torch.float32, L.F32), "f16": (torch.float16, L.F16), "bf16": (torch.bfloat16, L.BF16)}[dt]
     g = torch.Generator(device="cuda").manual_seed(n)
     b = (torch.randn((k, n), generator=g, device="cuda") * k ** -0.5).to(tdt)

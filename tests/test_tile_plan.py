@@ -74,7 +74,7 @@ def test_every_plan_has_an_estimate(plan, kind, k, rate):
 
 
 # (type, rows, K, N): skinny kernel against GEMV / engine in us, both timed
-FEW_ROWS = [("f16", 2, 768, 3072, 4.8, 5.2), ("f16", 2, 1024, 8192, 6.0, 7.2), ("f16", 16, 2048, 70001, 78.7, 85.5),
+FEW_ROWS = [("f16", 2, 768, 3072, 4.8, 5.2), ("f16", 2, 1024, 8192, 6.0, 7.2), ("f16", 16, 2048, 70001, 78.7, 85.5), ("f16", 8, 8192, 1100, 14.5, 16.4),
             ("f16", 8, 4096, 4096, 9.6, 30.2), ("f16", 9, 4096, 4096, 9.5, 11.7),
             ("f16", 32, 768, 768, 5.6, 8.1), ("f16", 24, 2048, 8192, 13.3, 11.7), ("f16", 32, 2048, 8192, 14.6, 12.4),
             ("f16", 24, 4096, 11008, 31.8, 22.3), ("f16", 32, 4096, 11008, 35.7, 22.7), ("f16", 24, 4096, 4096, 13.2, 12.3),
