@@ -1210,8 +1210,9 @@ extern "C" int ohip_gemm(ohip_ctx* ctx, const ohip_gemm_desc* d, const void* a, 
   const bool packed = !rows_direct(a, K, lda, eb, d->trans_a);
   TilePlan sc = M <= kMaxGemvM ? TilePlan{1, ctx->tile_override}
                                : plan_tiles(dense_kind(d->dtype), (int)N, (int)M, b->kc, ctx->tile_override);
+  const bool odd = !d->trans_a && (!aligned(a, 4) || (M > 1 && lda * eb % 4 != 0));
   const bool skinny = M <= kMaxSkinnyM && ctx->tile_override == 0 && !forced_splits() &&
-                      skinny_wins(d->dtype == OHIP_F32, M, N, b->kc, packed && !d->trans_a, sc);
+                      skinny_wins(d->dtype == OHIP_F32, M, N, b->kc, packed && !d->trans_a, odd, sc);
   const bool gemv = M <= kMaxGemvM && !skinny;
   if (skinny) sc = TilePlan{1, 0};
   if (sc.splits > 1 && scratch_frozen(ctx, ScratchPlan::rounded(split_ws_bytes((int)N, (int)M, sc.splits)) +

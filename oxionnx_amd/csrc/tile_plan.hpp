@@ -173,7 +173,9 @@ constexpr int kMaxSkinnyM = 32;
 // blocks of 16 weight rows each read the activations again, and a second
 // activation tile (over 16 rows) costs every weight byte more.  GEMV reads the
 // activations again for every weight row or two.  Rows that GEMV or the engine
-// would pack first cost them a launch (2.5); the engine's unsplit plans are
+// would pack first cost them a launch (2.5), and 16-bit rows at odd addresses
+// (not whole dwords) cost the skinny kernel's loads (8x3787x512 f16 10.6 us, 7.4
+// at K = 3788; 23x3787x1658 20.3 against 13.0 packed); the engine's unsplit plans are
 // 2 us slower at so few rows than at those its fit saw.  Fitted to 21 weights
 // of 256-70001 rows and 512-25088 columns at 2-32 rows, f16 and f32 (graph
 // replay), where both sides were timed: the choice is within 0.4 % of the
@@ -182,13 +184,14 @@ constexpr int kMaxSkinnyM = 32;
 // against 11.7).  5x768x3072 f16 6.6 -> 4.2 us, 8x4096x4096 36 -> 9.6, 9x4096x11008
 // 25.8 -> 21.5, f32 16x4096x4096 26 -> 21; 5x25088x512 f16 stays GEMV (11.3
 // against 34: 32 blocks).
-inline bool skinny_wins(bool f32, int64_t m, int64_t n, int64_t kc, bool pack, const TilePlan& engine) {
+inline bool skinny_wins(bool f32, int64_t m, int64_t n, int64_t kc, bool pack, bool odd, const TilePlan& engine) {
   const float steps = (float)((kc + 31) / 32), mb = (float)n * (float)kc * 16e-6f, rows = (float)m;
   const float acts = (float)((n + 15) / 16) * (float)kc * rows * 16e-6f;   // MB
   const float step = f32 ? .29f + .0125f * rows : .25f + .0115f * rows;
   const float rate = f32 ? (steps >= 8.0f ? 5.4f : 4.2f) : steps >= 16.0f ? 6.5f : steps >= 8.0f ? 5.4f : 4.6f;   // MB a us
   const float skinny =
-      std::max(step * steps, mb / rate) + acts * (f32 ? .01f : m > kMaxGemvM ? .05f : 0.0f) + (m > 16 ? mb * (f32 ? .2f : .12f) : 0.0f);
+      std::max(step * steps, mb / rate) + acts * (f32 ? .01f : m > kMaxGemvM ? .05f : 0.0f) + (m > 16 ? mb * (f32 ? .2f : .12f) : 0.0f) +
+      (odd ? .028f * steps * rows : 0.0f);
   const float other = m <= kMaxGemvM ? mb / 7.0f + rows * (.33f + (f32 ? .02f : m <= 2 ? .018f : .04f) * mb)
                                      : engine.us + (engine.splits == 1 ? 2.2f : 1.5f);
   return skinny < other + (pack ? 2.5f : 0.0f);

@@ -16,9 +16,9 @@ extern "C" float plan(int kind, int P, int Q, int kc, int forced, int batch, int
   out[1] = t.tile;
   return t.us;
 }
-extern "C" int skinny(int f32, int m, int n, int kc, int pack) {
+extern "C" int skinny(int f32, int m, int n, int kc, int pack, int odd) {
   const TilePlan t = m <= kMaxGemvM ? TilePlan{1, 0} : plan_tiles(f32 ? PlanKind::DenseF32 : PlanKind::Dense, n, m, kc, 0);
-  return skinny_wins(f32 != 0, m, n, kc, pack != 0, t);
+  return skinny_wins(f32 != 0, m, n, kc, pack != 0, odd != 0, t);
 }
 """
 
@@ -75,6 +75,8 @@ def test_every_plan_has_an_estimate(plan, kind, k, rate):
 
 # (type, rows, K, N): skinny kernel against GEMV / engine in us, both timed
 FEW_ROWS = [("f16", 2, 768, 3072, 4.8, 5.2), ("f16", 2, 1024, 8192, 6.0, 7.2), ("f16", 16, 2048, 70001, 78.7, 85.5), ("f16", 8, 8192, 1100, 14.5, 16.4),
+            ("f16", 23, 3787, 1658, 20.3, 13.0), ("f16", 23, 3788, 1658, 10.2, 13.0),
+            ("f16", 16, 2046, 512, 7.1, 10.3), ("f16", 8, 5001, 512, 12.8, 9.9), ("f16", 8, 3787, 1658, 11.1, 18.7),
             ("f16", 8, 4096, 4096, 9.6, 30.2), ("f16", 9, 4096, 4096, 9.5, 11.7),
             ("f16", 32, 768, 768, 5.6, 8.1), ("f16", 24, 2048, 8192, 13.3, 11.7), ("f16", 32, 2048, 8192, 14.6, 12.4),
             ("f16", 24, 4096, 11008, 31.8, 22.3), ("f16", 32, 4096, 11008, 35.7, 22.7), ("f16", 24, 4096, 4096, 13.2, 12.3),
@@ -88,7 +90,8 @@ FEW_ROWS = [("f16", 2, 768, 3072, 4.8, 5.2), ("f16", 2, 1024, 8192, 6.0, 7.2), (
 def test_few_rows_take_the_faster_kernel(lib, case):
     dt, m, k, n, skinny, other = case
     per = 4 if dt == "f32" else 8
-    assert bool(lib.skinny(int(dt == "f32"), m, n, -(-k // per), int(k % per != 0))) == (skinny < other)
+    odd = dt == "f16" and k % 2   # rows at odd addresses
+    assert bool(lib.skinny(int(dt == "f32"), m, n, -(-k // per), int(k % per != 0), odd)) == (skinny < other)
 
 
 # (kind, elements a chunk, rows, K, N): us by K slices (1: the fastest tile unsplit)
