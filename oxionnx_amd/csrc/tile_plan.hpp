@@ -53,13 +53,13 @@ enum class PlanKind { Dense, DenseF32, Conv };   // f16 / bf16 / int8 rows; f32 
 // reduction's launch also costs the host about 1.5 us, which is in its fixed
 // term whether or not a host waits: a capture has to plan as the eager call
 // before it did, for the same scratch and the same bits).  The slices of the
-// other kinds are fitted to 104 products of 33-600 rows timed on 2-16 slices,
-// eager and by replay (their mean), by the loss of the choice: 0.2 % in the
-// mean for f32 (1.8 % at most), 0.9 % for f16 and int8 (7 %).  Every count up
-// to ten is a candidate there: 48 blocks of f32 200x2048x768 fill a round with
-// five slices (16.7 us; four 18.3, six 19.5).  Against rules on the number of
-// blocks: f16 1024x1024x768 13.7 -> 9.0 us (split, now unsplit), 1500x1024x2048
-// 18.0 -> 12.7, 838x2688x2880 37 -> 24.
+// other kinds are fitted to 244 products of 33-1500 rows timed on 2-16 slices,
+// eager and by replay (their mean), by the loss of the choice: 0.3 % in the
+// mean for f32 (4 % at most), 0.9 % for f16 (10 %) and 1.7 % for int8 (9 %).
+// Every count up to ten is a candidate there: 48 blocks of f32 200x2048x768
+// fill a round with five slices (16.7 us; four 18.3, six 19.5).  Against rules
+// on the number of blocks: f16 1024x1024x768 13.7 -> 9.0 us (split, now
+// unsplit), 1500x1024x2048 18.0 -> 12.7, 838x2688x2880 37 -> 24.
 // Grids of a round of 256x256 tiles and a long K take tile 16 outright: its
 // advantage there is the clock and the cache, which the stages' cost does
 // not show (4096x4096x11008 f16 291 us against 324 on tiles 3, 4 and 18).
@@ -86,8 +86,8 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
   static constexpr TileCost kConv[] = {{1, 64, 64, 4, .522f, .234f, 1.17f},   {9, 64, 64, 2, .386f, .254f, 1.17f},
                                        {8, 128, 128, 2, .633f, .403f, 1.56f}, {12, 128, 128, 1, .510f, .510f, 2.15f},
                                        {3, 256, 128, 1, .708f, .708f, 4.0f},  {4, 128, 256, 1, .708f, .708f, 4.0f}};
-  const ReduceCost red = kind == PlanKind::Dense      ? ReduceCost{1.5f, .35f, .18f}
-                         : kind == PlanKind::DenseF32 ? ReduceCost{2.0f, .50f, .03f}
+  const ReduceCost red = kind == PlanKind::Dense      ? ReduceCost{1.5f, .50f, .14f}
+                         : kind == PlanKind::DenseF32 ? ReduceCost{2.0f, .40f, .14f}
                                                       : ReduceCost{1.21f + 1.5f, .321f, .121f};
   const TileCost* tab = kind == PlanKind::Dense ? kDense : kind == PlanKind::DenseF32 ? kF32 : kConv;
   const int ntab = kind == PlanKind::Dense      ? (int)(sizeof(kDense) / sizeof(TileCost))
@@ -131,7 +131,14 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     const int64_t nb = blocks(t.bp, t.bq);
     const float c = time(t, nb, nk);
     if (c < cost) { cost = c; best = {1, t.id}; }
-    if (!may_split || (t.id != 9 && t.id != 8)) continue;
+  }
+  // (products of few stages: a reduction's launch costs a waiting host more
+  // than the slices gain, f16 165x768x128 eager 7.2 us, 8.4 in four slices)
+  const bool split = may_split && (kind == PlanKind::Conv || cost >= 4.6f);
+  for (int i = 0; split && i < ntab; ++i) {
+    const TileCost& t = tab[i];
+    if (t.id != 9 && t.id != 8) continue;
+    const int64_t nb = blocks(t.bp, t.bq);
     const float mb = (float)P * (float)Q * (float)batch * 4e-6f;
     // (each count a constant: small eager calls wait for this)
     auto slices = [&](auto count) {

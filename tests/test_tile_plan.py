@@ -103,6 +103,8 @@ SPLITS = [((1, 4, 128, 768, 3072), {1: 20.2, 2: 15.6, 3: 18.0, 4: 16.8, 5: 16.7,
           ((1, 4, 156, 6864, 1074), {1: 149.6, 5: 37.4, 8: 39.0, 9: 36.8, 10: 35.0, 12: 42.9}),
           ((1, 4, 256, 768, 3072), {1: 21.0, 2: 23.2, 3: 26.8, 4: 23.5, 5: 24.8}),
           ((0, 8, 128, 768, 3072), {1: 7.4, 2: 9.0, 3: 10.3, 4: 10.8}),
+          ((0, 8, 148, 1331, 2336), {1: 12.9, 2: 12.8, 3: 14.0, 4: 14.7}),
+          ((0, 8, 165, 768, 128), {1: 6.8, 2: 8.3, 3: 8.4, 4: 8.2}),   # (eager; by replay 7.1, 7.4, 6.9, 6.7)
           ((0, 8, 128, 8192, 4096), {1: 57.9, 3: 26.2, 4: 23.7, 5: 28.2, 8: 28.3}),
           ((0, 16, 300, 2048, 512), {1: 10.1, 2: 9.6, 3: 9.2, 4: 8.8, 5: 9.5, 6: 9.5, 8: 10.3}),
           ((0, 16, 206, 1931, 159), {1: 13.1, 2: 12.0, 3: 11.4, 4: 10.8, 5: 11.3, 6: 11.1, 8: 10.9, 12: 11.5})]
