@@ -79,7 +79,8 @@ int ohip_sync(ohip_ctx* ctx);
  * on the context's stream; every dispatch until ohip_graph_end is recorded,
  * not run.  Dispatches must already be warm (weights, constants, scratch and
  * output tables), because uploads, allocations and synchronisations cannot be
- * captured; a call that can do without missing scratch (unsplit) does.
+ * captured; a call that can do without missing scratch (unsplit, in place,
+ * or a fused norm in two steps) does.
  * While a capture is open, freed device buffers are parked for the graph,
  * which keeps them until ohip_graph_destroy; a replay writes the same
  * buffers, so the caller keeps the captured inputs and outputs alive and

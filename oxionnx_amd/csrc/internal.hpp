@@ -186,7 +186,7 @@ hipError_t run_dense_quant(const DenseOperand& x, const DenseOperand& y, const Q
 hipError_t run_conv_quant(const Im2colOperand& col, const DenseOperand& w, bool col_on_x, const QuantOut& o,
                           int tile, hipStream_t st);
 hipError_t run_gemv(int dtype, const GemvArgs& g, const FloatOut& o, hipStream_t st);
-// 2 to 32 rows (skinny_kernel) of K elements, of any stride and alignment;
+// 1 to 32 rows (skinny_kernel) of K elements, of any stride and alignment;
 // zero16: 16 zero bytes in device memory
 hipError_t run_skinny(int dtype, const GemvArgs& g, int K, const void* zero16, const FloatOut& o, hipStream_t st);
 // Direct (non-MFMA) grouped convolution; see conv_direct_kernel.

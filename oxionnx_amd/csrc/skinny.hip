@@ -1,5 +1,5 @@
 // Products of a few activation rows with a packed weight: Gemm with 2 to 32
-// rows (a batch of faces, a decode batch).
+// rows (a batch of faces, a decode batch), and of one misaligned row.
 #include "launch.hpp"
 
 namespace ohip {
