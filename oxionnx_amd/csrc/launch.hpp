@@ -585,12 +585,6 @@ inline hipError_t launch_unsplit(const LX& lx, const LY& ly, const Epi& epi, int
     default: return launch_tile<O, XX, XY, T64>(lx, ly, epi, P, Q, kc, st);
   }
 }
-template <Op O, bool XX, bool XY, class LX, class LY, class Epi>
-inline hipError_t launch_any(const LX& lx, const LY& ly, const Epi& epi, int P, int Q, int kc, int tile,
-                             int splits, void* split_ws, hipStream_t st) {
-  if (splits > 1) return launch_split<O, XX, XY>(lx, ly, epi, P, Q, kc, tile, splits, split_ws, st);
-  return launch_unsplit<O, XX, XY>(lx, ly, epi, P, Q, kc, tile, st);
-}
 
 // Per-slice pads (Im2colNHWC::zpt / zpl) hold four entries, indexed by the
 // batch slice: a launch that uses them must have at most four slices and no
