@@ -132,9 +132,12 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
     const float c = time(t, nb, nk);
     if (c < cost) { cost = c; best = {1, t.id}; }
   }
-  // (products of few stages: a reduction's launch costs a waiting host more
-  // than the slices gain, f16 165x768x128 eager 7.2 us, 8.4 in four slices)
-  const bool split = may_split && (kind == PlanKind::Conv || cost >= 4.6f);
+  // Few stages: a reduction's launch costs a waiting host more than the slices
+  // gain (f16 165x768x128 eager 7.2 us, 8.4 in four slices; of a batch, which a
+  // transposing launch precedes, f32 5 x 16x238x180 14.6 and 16.1; staged f16
+  // convolutions 2x32x8x8 -> 144 5x5 12.6 and 14.1)
+  const bool split = may_split && cost >= (kind == PlanKind::Conv ? 6.3f : 4.6f);
+  const float launch = kind != PlanKind::Conv && batch > 1 ? 1.0f : 0.0f;
   for (int i = 0; split && i < ntab; ++i) {
     const TileCost& t = tab[i];
     if (t.id != 9 && t.id != 8) continue;
@@ -146,7 +149,7 @@ inline TilePlan plan_tiles(PlanKind kind, int P, int Q, int kc, int override_til
       const uint32_t per = ((uint32_t)nk + most - 1) / most;
       if (per < 2) return false;
       const int s = per * (most - 1) < (uint32_t)nk ? (int)most : filled(most);
-      const float cs = time(t, nb * s, per) + red.fix + red.per_slice * (float)s + red.per_mb * mb * (float)s;
+      const float cs = time(t, nb * s, per) + red.fix + launch + red.per_slice * (float)s + red.per_mb * mb * (float)s;
       if (cs < cost) { cost = cs; best = {s, t.id == 9 ? 10 : 11}; }
       return true;
     };
